@@ -8,15 +8,13 @@
 //
 //   rmsnorm / enc_aux_norm      one workgroup per row (or row chunk)
 //   qk_norm_rope                one wavefront per (row, head)
-//   attention (head_dim 128)    flash-decoding: one workgroup per (kv head, 64
-//                               positions); the 64 queries of a kv head (m tokens x
-//                               n_q/n_kv heads) against the chunk's keys and values
-//                               with v_mfma_f32_16x16x32_bf16, every f32 operand split
-//                               exactly into three bf16 parts and the six significant
-//                               part products accumulated (f32-grade); per-chunk
-//                               maxima, sums and partial outputs merged by a second
-//                               kernel
-//   attention (other head_dim)  one wavefront per (row, head), online softmax
+//   attention                   head_dim 128, up to 64 queries per kv head: 16 queries of
+//                               a kv head per workgroup over a run of the sequence, on f16
+//                               parts (k_attn_split), or, for a few queries, dots from
+//                               memory (k_attn_decode, k_attn_token) and a combine; more
+//                               queries, and head_dim 64 and 256: blocks of 64 queries
+//                               over f16 parts staged in LDS (k_attn_rows); other head
+//                               sizes: one wavefront per (row, head), online softmax
 //   softplus gate, add          elementwise
 #include <cmath>
 #include <cstring>
@@ -1099,7 +1097,410 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
     }
 }
 
-// Any head_dim <= 256: one wavefront per (row, q head), online softmax as mha_attn.comp.
+// Many queries of one kv head (more than AQ), or a head size other than AHD: HD 64, 128
+// or 256.  Workgroup (kv head h, query block qg, chunk c): wavefront w takes queries 64 qg
+// + 16 w .. + 15 of kv head h over chunk c of the 32-position tiles that the block can
+// see, so that each K and V element is read and split once per 64 queries.
+//
+//   K     wavefront w loads rows 8w .. 8w+7 of the tile (8 lanes a row), scales each row
+//         by the power of two 2^e that puts its largest magnitude in [2^14, 2^15) and
+//         stores its f16 parts (f16_parts2) row by row to LDS, with 2^-e;
+//   V     wavefront w loads positions 4w + i and 16 + 4w + i (i < 4), scales by 2^8, and
+//         stores the f16 parts transposed (per dim, 8 positions a 16-byte word), in the
+//         order in which a lane group holds the probabilities of those positions;
+//   S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, each three products of
+//         the parts (hi hi + hi lo + lo hi); queries scaled as K rows are.
+//
+// The tile after the next one is loaded into registers, the next one converted into the
+// other LDS buffer, while the current one is multiplied: one barrier per tile.  A tile
+// with a non-finite K or V or a K magnitude (or queries) of 65504 and above (whose row's
+// other elements the f16 parts would lose), or whose V lies outside [2^-12, 2^8) by its
+// largest magnitude, takes that product element by element in f32 from memory (masked
+// positions skipped, so that what lies past the causal limit never reaches a result).
+//
+// One wavefront per (row, q head) over the whole sequence (k_attn_simple) reads K and V
+// once per query, one position at a time, and is bound by that chain: 32 rows of 32 / 8
+// heads over 4096 positions 6880 us, here 31 (about 25 and 5.5 for the merge: the loads of
+// the first tiles, eight tiles a workgroup and K and V twice through the L2, one for each
+// 64 of the 128 queries).
+constexpr uint32_t RQB = 64, RPT = 32;  // queries per workgroup, positions per tile
+constexpr uint32_t RVS = RPT + 8;       // halves per dim of the V tile: 16-byte reads of 16 dims on distinct banks
+
+template <int HD>
+struct RowsLds {
+    static constexpr uint32_t KS = HD + 8;  // halves per K row, likewise
+    _Float16 k[2][2][RPT * KS];             // [buffer][hi, lo]
+    _Float16 v[2][2][HD * RVS];
+    float ke[2][RPT];   // 2^-e of the K rows
+    float vmx[2][4];    // largest |V| of each wavefront's share (NaN: a NaN among them)
+    uint32_t kbad[2][4];
+};
+
+struct RowsAttn {
+    const float *q, *k0, *v0, *k1, *v1;
+    uint32_t n0, S, rows, n_q, n_kv, qpos0, ngq, nch;
+    int causal, gmode;
+    float scale;
+    float *part_o, *part_ml;  // nch > 1: [group][chunk][64][HD] and [group][chunk][64][2]
+    float *out;
+    const float *gate;
+};
+
+// 2^e that puts a (finite, nonzero) magnitude in [2^14, 2^15); 1 for zero and non-finite
+__device__ __forceinline__ int scale_exp(float amax) {
+    if (!(amax > 0.0f && amax <= 3.4028234664e38f)) return 0;
+    const int e = 15 - __builtin_amdgcn_frexp_expf(amax);
+    return e < -126 ? -126 : (e > 126 ? 126 : e);
+}
+
+__device__ __forceinline__ float attn_gate(float gv, int gmode) {
+    return gmode == 2 ? logf(1.0f + expf(gv)) : softplus_gate(gv);
+}
+
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
+    constexpr int J = HD / 32, DT = HD / 16, KV4 = HD / 32;  // k steps, dim tiles, float4s of K per thread
+    constexpr int DPT = HD / 64;                             // V dims per thread
+    constexpr int SETS = HD <= 128 ? 2 : 1;                  // tiles ahead in registers (256: the register budget)
+    constexpr uint32_t KS = RowsLds<HD>::KS;
+    extern __shared__ __attribute__((aligned(16))) uint8_t rows_lds[];
+    RowsLds<HD> &L = *reinterpret_cast<RowsLds<HD> *>(rows_lds);
+    const uint32_t id = blockIdx.x, slot = id / 8;
+    const uint32_t qg = a.ngq - 1 - slot % a.ngq, r = (slot / a.ngq) * 8 + id % 8;  // the longest causal blocks first
+    if (r >= a.n_kv * a.nch) return;  // uniform over the workgroup
+    const uint32_t h = r / a.nch, c = r % a.nch;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, kg = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t G = a.n_q / a.n_kv, nq = a.rows * G, kvld = a.n_kv * HD;
+    const float neg1 = neg_one();
+    auto kvrow = [&](const float *b0, const float *b1, uint32_t p) {  // positions past S read row S - 1 (masked)
+        const uint32_t pc = p < a.S ? p : a.S - 1;
+        return (pc < a.n0 ? b0 + (uint64_t)pc * kvld : b1 + (uint64_t)(pc - a.n0) * kvld) + h * HD;
+    };
+    // the positions this block can see, its tiles, and this chunk's share of them
+    const uint32_t qlast = RQB * qg + RQB - 1 < nq ? RQB * qg + RQB - 1 : nq - 1;
+    const uint32_t end = a.causal && a.qpos0 + qlast / G + 1 < a.S ? a.qpos0 + qlast / G + 1 : a.S;
+    const uint32_t nt = (end + RPT - 1) / RPT, tb = attn_tile0(c, nt, a.nch), te = attn_tile0(c + 1, nt, a.nch);
+
+    typedef float vdims __attribute__((ext_vector_type(DPT)));
+    f32x4 kr[SETS][KV4];  // native vectors: arrays of HIP's float4 do not always stay in registers
+    vdims vr[SETS][8];
+    auto f4 = [](const f32x4 &v) { return make_float4(v[0], v[1], v[2], v[3]); };
+    auto load = [&](int s, uint32_t tile) __attribute__((always_inline)) {
+        const float *kp = kvrow(a.k0, a.k1, RPT * tile + 8 * wave + (lane >> 3)) + 8 * (lane & 7u);
+#pragma unroll
+        for (int j = 0; j < KV4; j++) kr[s][j] = *reinterpret_cast<const f32x4 *>(kp + 64 * (j >> 1) + 4 * (j & 1));
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float *vp = kvrow(a.v0, a.v1, RPT * tile + (i >> 2) * 16 + 4 * wave + (i & 3)) + DPT * lane;
+            vr[s][i] = *reinterpret_cast<const vdims *>(vp);
+        }
+    };
+    auto convert = [&](int s, int b) __attribute__((always_inline)) {
+        // K: row 8 wave + lane / 8, dims 64 j + 8 (lane % 8) .. + 7
+        float mx = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KV4; j += 2) mx = absmax8(mx, f4(kr[s][j]), f4(kr[s][j + 1]));
+        mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0xB1, 0xF, 0xF, false)));
+        mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x4E, 0xF, 0xF, false)));
+        mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x141, 0xF, 0xF, false)));
+        // x - x is 0 unless x is infinite or NaN (v_max3 may drop a NaN)
+        float nf = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KV4; j++) {
+            const float4 f = f4(kr[s][j]);
+            nf += ((f.x - f.x) + (f.y - f.y)) + ((f.z - f.z) + (f.w - f.w));
+        }
+        const int e = scale_exp(mx);
+        const uint32_t row = 8 * wave + (lane >> 3);
+#pragma unroll
+        for (int j = 0; j < KV4; j += 2) {
+            float4 x = f4(kr[s][j]), y = f4(kr[s][j + 1]);
+            x = make_float4(__builtin_ldexpf(x.x, e), __builtin_ldexpf(x.y, e), __builtin_ldexpf(x.z, e),
+                            __builtin_ldexpf(x.w, e));
+            y = make_float4(__builtin_ldexpf(y.x, e), __builtin_ldexpf(y.y, e), __builtin_ldexpf(y.z, e),
+                            __builtin_ldexpf(y.w, e));
+            f16x8 hi, lo;
+            f16_parts8(x, y, neg1, hi, lo);
+            const uint32_t o = row * KS + 32 * j + 8 * (lane & 7u);
+            *reinterpret_cast<f16x8 *>(&L.k[b][0][o]) = hi;
+            *reinterpret_cast<f16x8 *>(&L.k[b][1][o]) = lo;
+        }
+        if ((lane & 7u) == 0) L.ke[b][row] = __builtin_ldexpf(1.0f, -e);
+        const uint64_t kb = __builtin_amdgcn_ballot_w64(nf != 0.0f || !(mx < 65504.0f));
+        // V: dims DPT lane .. of this wavefront's eight positions
+        float vm = 0.0f, vn = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DPT; d++) {
+            float4 x = make_float4(vr[s][0][d], vr[s][1][d], vr[s][2][d], vr[s][3][d]);
+            float4 y = make_float4(vr[s][4][d], vr[s][5][d], vr[s][6][d], vr[s][7][d]);
+            vm = absmax8(vm, x, y);
+            vn += (((x.x - x.x) + (x.y - x.y)) + ((x.z - x.z) + (x.w - x.w))) +
+                  (((y.x - y.x) + (y.y - y.y)) + ((y.z - y.z) + (y.w - y.w)));
+            x = make_float4(x.x * 256.0f, x.y * 256.0f, x.z * 256.0f, x.w * 256.0f);
+            y = make_float4(y.x * 256.0f, y.y * 256.0f, y.z * 256.0f, y.w * 256.0f);
+            f16x8 hi, lo;
+            f16_parts8(x, y, neg1, hi, lo);
+            const uint32_t o = (DPT * lane + d) * RVS + 8 * wave;
+            *reinterpret_cast<f16x8 *>(&L.v[b][0][o]) = hi;
+            *reinterpret_cast<f16x8 *>(&L.v[b][1][o]) = lo;
+        }
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) vm = fmaxf(vm, __shfl_xor(vm, o));
+        const uint64_t vb = __builtin_amdgcn_ballot_w64(vn != 0.0f);
+        if (lane == 0) {
+            L.kbad[b][wave] = kb ? 1u : 0u;
+            L.vmx[b][wave] = vb ? INFINITY : vm;
+        }
+    };
+
+    // this lane's query: k step j, dims 32 j + 8 kg .. + 7 (a dead query column repeats the
+    // last one; its results are not stored)
+    const uint32_t qi = RQB * qg + 16 * wave + l16;
+    const bool wlive = RQB * qg + 16 * wave < nq, qlive = qi < nq;  // wlive: uniform over the wavefront
+    const uint32_t qc = qlive ? qi : nq - 1, qt = qc / G, qpos = a.qpos0 + qt;
+    const float *qp = a.q + (uint64_t)qt * a.n_q * HD + (uint64_t)(h * G + qc % G) * HD;
+    f16x8 qh[J], ql[J];
+    float qs;
+    bool qbad;
+    if (tb < te) load(0, tb);
+    if constexpr (SETS == 2)
+        if (tb < te) load(1, tb + 1 < te ? tb + 1 : tb);
+    {
+        float4 f[2 * J];
+        float mx = 0.0f, nf = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            f[2 * j] = *reinterpret_cast<const float4 *>(qp + 32 * j + 8 * kg);
+            f[2 * j + 1] = *reinterpret_cast<const float4 *>(qp + 32 * j + 8 * kg + 4);
+            mx = absmax8(mx, f[2 * j], f[2 * j + 1]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2 * J; j++) nf += ((f[j].x - f[j].x) + (f[j].y - f[j].y)) + ((f[j].z - f[j].z) + (f[j].w - f[j].w));
+        qbad = __builtin_amdgcn_ballot_w64(nf != 0.0f || !(mx < 65504.0f)) != 0;
+        mx = rows4_max(mx);
+        const int e = scale_exp(mx);
+#pragma unroll
+        for (int j = 0; j < 2 * J; j++)
+            f[j] = make_float4(__builtin_ldexpf(f[j].x, e), __builtin_ldexpf(f[j].y, e), __builtin_ldexpf(f[j].z, e),
+                               __builtin_ldexpf(f[j].w, e));
+#pragma unroll
+        for (int j = 0; j < J; j++) f16_parts8(f[2 * j], f[2 * j + 1], neg1, qh[j], ql[j]);
+        qs = __builtin_ldexpf(a.scale * 1.44269504088896341f, -e);  // scores in base-2 units
+    }
+    const float qs1 = a.scale * 1.44269504088896341f;
+    f32x4 Od[DT];
+#pragma unroll
+    for (int t = 0; t < DT; t++) Od[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, lsum = 0.0f;
+    // positions 16 pt + 4 kg + i of the tile against the lane's query
+    auto compute = [&](int b, uint32_t tile) __attribute__((always_inline)) {
+        const uint32_t p0 = RPT * tile + 4 * kg;
+        bool ok[2][4];
+        float sv[2][4], tmax = -INFINITY;
+#pragma unroll
+        for (int pt = 0; pt < 2; pt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t p = p0 + 16 * pt + i;
+                ok[pt][i] = p < a.S && (!a.causal || p <= qpos);
+            }
+        const uint32_t kbad = (L.kbad[b][0] | L.kbad[b][1]) | (L.kbad[b][2] | L.kbad[b][3]);
+        if (!qbad && __builtin_amdgcn_readfirstlane(kbad) == 0) {
+            f32x4 sc[2][2];
+#pragma unroll
+            for (int pt = 0; pt < 2; pt++)
+#pragma unroll
+                for (int u = 0; u < 2; u++) sc[pt][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int pt = 0; pt < 2; pt++) {
+                    const uint32_t o = (16 * pt + l16) * KS + 32 * j + 8 * kg;
+                    const f16x8 kh = *reinterpret_cast<const f16x8 *>(&L.k[b][0][o]);
+                    const f16x8 kl = *reinterpret_cast<const f16x8 *>(&L.k[b][1][o]);
+                    f32x4 &s = sc[pt][j & 1];
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[j], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[j], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[j], s, 0, 0, 0);
+                    if constexpr (HD > 128) __builtin_amdgcn_sched_barrier(0);  // fragments read as used: no spills
+                }
+#pragma unroll
+            for (int pt = 0; pt < 2; pt++) {
+                const float4 ke = *reinterpret_cast<const float4 *>(&L.ke[b][16 * pt + 4 * kg]);
+                const float kx[4] = {ke.x, ke.y, ke.z, ke.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) sv[pt][i] = (sc[pt][0][i] + sc[pt][1][i]) * (kx[i] * qs);
+            }
+        } else {
+#pragma unroll
+            for (int pt = 0; pt < 2; pt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float *kp = kvrow(a.k0, a.k1, p0 + 16 * pt + i);
+                    float d = 0.0f;
+                    if (ok[pt][i])
+                        for (uint32_t e = 0; e < (uint32_t)HD; e++) d = __builtin_fmaf(qp[e], kp[e], d);
+                    sv[pt][i] = d * qs1;
+                }
+        }
+#pragma unroll
+        for (int pt = 0; pt < 2; pt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                sv[pt][i] = ok[pt][i] ? sv[pt][i] : -INFINITY;
+                tmax = fmaxf(tmax, sv[pt][i]);
+            }
+        tmax = rows4_max(tmax);
+        const float mn = fmaxf(m, tmax), mu = mn == -INFINITY ? 0.0f : mn;
+        if (__builtin_amdgcn_ballot_w64(mn != m)) {  // some query's max moved: rescale (2^-inf = 0)
+            const float f = __builtin_amdgcn_exp2f(m - mu);
+            lsum *= f;
+#pragma unroll
+            for (int t = 0; t < DT; t++) Od[t] *= f;
+        }
+        m = mn;
+        float pv[8];
+#pragma unroll
+        for (int pt = 0; pt < 2; pt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                pv[4 * pt + i] = __builtin_amdgcn_exp2f(sv[pt][i] - mu);
+                lsum += pv[4 * pt + i];
+            }
+        const float vm = fmaxf(fmaxf(L.vmx[b][0], L.vmx[b][1]), fmaxf(L.vmx[b][2], L.vmx[b][3]));
+        if (__builtin_amdgcn_ballot_w64(vm >= 0x1p-12f && vm < 255.875f)) {  // uniform
+            f16x8 ph, pl;
+            f16_parts8(make_float4(pv[0], pv[1], pv[2], pv[3]), make_float4(pv[4], pv[5], pv[6], pv[7]), neg1, ph, pl);
+#pragma unroll
+            for (int t = 0; t < DT; t++) {
+                const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
+                const f16x8 vh = *reinterpret_cast<const f16x8 *>(&L.v[b][0][o]);
+                const f16x8 vl = *reinterpret_cast<const f16x8 *>(&L.v[b][1][o]);
+                f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl, x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph, x, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i], 0x1p-8f, Od[t][i]);
+                if constexpr (HD > 128)
+                    if (t & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for (uint32_t j = 0; j < RPT; j++) {  // the tile's positions: lane group j / 4 % 4, its weight 4 (j / 16) + j % 4
+                const uint32_t e = 4 * (j >> 4) + (j & 3u);
+                float w = pv[0];
+#pragma unroll
+                for (uint32_t i = 1; i < 8; i++) w = e == i ? pv[i] : w;
+                w = __shfl(w, (int)(16 * ((j >> 2) & 3u) + l16));
+                const uint32_t p = RPT * tile + j;
+                const bool live = p < a.S && (!a.causal || p <= qpos);
+                const float *vp = kvrow(a.v0, a.v1, p) + 4 * kg;
+#pragma unroll
+                for (int t = 0; t < DT; t++) {
+                    const float4 f = *reinterpret_cast<const float4 *>(vp + 16 * t);
+                    if (live) {
+                        Od[t][0] = __builtin_fmaf(w, f.x, Od[t][0]);
+                        Od[t][1] = __builtin_fmaf(w, f.y, Od[t][1]);
+                        Od[t][2] = __builtin_fmaf(w, f.z, Od[t][2]);
+                        Od[t][3] = __builtin_fmaf(w, f.w, Od[t][3]);
+                    }
+                }
+            }
+        }
+    };
+    // a wavefront skips tiles that none of its queries sees
+    const uint32_t wq = RQB * qg + 16 * wave + 15 < nq ? RQB * qg + 16 * wave + 15 : nq - 1;
+    const uint32_t wend = a.causal ? a.qpos0 + wq / G + 1 : a.S;
+    auto step = [&](int s, int b, uint32_t tile) __attribute__((always_inline)) {  // buffer b holds `tile`, set s the next one
+        if (wlive && RPT * tile < wend) compute(b, tile);
+        if constexpr (HD > 128) __builtin_amdgcn_sched_barrier(0);
+        if (tile + 1 < te) {
+            convert(s, b ^ 1);
+            if constexpr (HD > 128) __builtin_amdgcn_sched_barrier(0);
+            load(s, tile + 1 + SETS < te ? tile + 1 + SETS : te - 1);
+        }
+        __syncthreads();
+    };
+    if (tb < te) {
+        convert(0, 0);
+        load(0, tb + SETS < te ? tb + SETS : te - 1);
+        __syncthreads();
+        for (uint32_t t = tb; t < te; t += 2) {
+            step(SETS - 1, 0, t);
+            if (t + 1 >= te) break;  // uniform
+            step(0, 1, t + 1);
+        }
+    }
+    lsum = lane_add_x32(lane_add_x16(lsum));
+    if (!wlive) return;
+    if (a.nch > 1) {
+        const uint64_t pi = ((uint64_t)(h * a.ngq + qg) * a.nch + c) * RQB + 16 * wave + l16;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+            *reinterpret_cast<float4 *>(a.part_o + pi * HD + 16 * t + 4 * kg) =
+                make_float4(Od[t][0], Od[t][1], Od[t][2], Od[t][3]);
+        if (kg == 0) *reinterpret_cast<float2 *>(a.part_ml + 2 * pi) = make_float2(m, lsum);
+        return;
+    }
+    if (!qlive) return;
+    const uint32_t hq = h * G + qi % G;
+    const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+    const float g = a.gate ? attn_gate(a.gate[(uint64_t)qt * a.n_q + hq], a.gmode) : 1.0f;
+    float *op = a.out + ((uint64_t)qt * a.n_q + hq) * HD + 4 * kg;
+#pragma unroll
+    for (int t = 0; t < DT; t++) {
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] = lsum > 0.0f ? (Od[t][i] * inv) * g : 0.0f;
+        *reinterpret_cast<float4 *>(op + 16 * t) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// The chunks of k_attn_rows merged, one wavefront per (row, q head), lane l dims l, l +
+// 64, ...: every chunk's max and sum in one load (lane c: chunk c, at most 64), then the
+// chunks' outputs in chunk order, eight in flight.
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_rows_merge(RowsAttn a) {
+    constexpr int DPT = HD / 64;
+    const uint32_t lane = threadIdx.x & 63u, u = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (u >= a.rows * a.n_q) return;
+    const uint32_t t = u / a.n_q, hq = u % a.n_q, G = a.n_q / a.n_kv, h = hq / G, qi = t * G + hq % G;
+    const uint64_t p0 = (uint64_t)(h * a.ngq + qi / RQB) * a.nch * RQB + qi % RQB;
+    const uint32_t cl = lane < a.nch ? lane : a.nch - 1;
+    const float2 ml = *reinterpret_cast<const float2 *>(a.part_ml + 2 * (p0 + (uint64_t)cl * RQB));
+    const float mc = lane < a.nch ? ml.x : -INFINITY;
+    float M = mc;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    const float w = mc == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc - M);
+    const float l = wave_sum(w * ml.y);
+    float o[DPT];
+#pragma unroll
+    for (int d = 0; d < DPT; d++) o[d] = 0.0f;
+    for (uint32_t c0 = 0; c0 < a.nch; c0 += 8) {
+        float v[8][DPT];
+#pragma unroll
+        for (uint32_t b = 0; b < 8; b++) {
+            const uint32_t c = c0 + b < a.nch ? c0 + b : a.nch - 1;
+#pragma unroll
+            for (int d = 0; d < DPT; d++) v[b][d] = a.part_o[(p0 + (uint64_t)c * RQB) * HD + 64 * d + lane];
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < 8; b++) {
+            const float wc = __shfl(w, (int)(c0 + b < 64 ? c0 + b : 63u));
+#pragma unroll
+            for (int d = 0; d < DPT; d++) o[d] = c0 + b < a.nch ? __builtin_fmaf(wc, v[b][d], o[d]) : o[d];
+        }
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float g = a.gate ? attn_gate(a.gate[(uint64_t)t * a.n_q + hq], a.gmode) : 1.0f;
+    float *op = a.out + ((uint64_t)t * a.n_q + hq) * HD;
+#pragma unroll
+    for (int d = 0; d < DPT; d++) op[64 * d + lane] = l > 0.0f ? (o[d] * inv) * g : 0.0f;
+}
+
+// Any other head_dim <= 256 (and unaligned operands): one wavefront per (row, q head),
+// online softmax as mha_attn.comp.
 __global__ __launch_bounds__(256) void k_attn_simple(const float *__restrict__ q, const float *__restrict__ k0,
                                                      const float *__restrict__ v0, uint32_t n0,
                                                      const float *__restrict__ k1, const float *__restrict__ v1,
@@ -1229,17 +1630,69 @@ uint32_t attn_split_chunks(uint32_t S, uint32_t groups) {
 // zero between calls), then the partials of whichever kernel runs.
 uint32_t attn_cnt_floats(uint32_t n_kv) { return (4 * n_kv + 63) / 64 * 64; }
 
-size_t attn_partial_floats(uint32_t S, uint32_t n_kv) {
+// k_attn_rows: head sizes it is built for; more than AQ queries per kv head of AHD (up to
+// there k_attn_split and the few-query kernels), any number of the other sizes.
+bool attn_rows_ok(uint32_t S, uint32_t queries, uint32_t hd) {
+    return S && (hd == AHD ? queries > AQ : hd == 64 || hd == 256);
+}
+
+// Chunks per (kv head, 64-query block) of k_attn_rows: about one workgroup per CU, down to
+// one tile a chunk.  us for four layers, against the alternatives: 32 rows of 32 / 8 heads
+// of 128 over 4096 positions 123 (two workgroups per CU: 138; k_attn_simple 27530); 16 rows
+// of 16 / 4 heads of 256 over 2000 96 (at least two tiles a chunk: 99); 32 rows of 4 / 1
+// heads of 128 over 300 45 (51).
+uint32_t rows_chunks(uint32_t S, uint32_t groups) {
+    const uint32_t nt = (S + RPT - 1) / RPT, cus = (uint32_t)device_cus();
+    const uint32_t per = cus / groups;
+    uint32_t nch = per < nt ? per : nt;
+    nch = nch < 64 ? nch : 64;  // k_attn_rows_merge: a chunk a lane
+    return nch ? nch : 1;
+}
+
+// Floats of k_attn_rows's partials (0: one chunk, nothing to merge).
+size_t rows_partial_floats(uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_kv, uint32_t hd) {
+    const uint64_t nq = (uint64_t)rows * (n_q / n_kv), groups = n_kv * ((nq + RQB - 1) / RQB);
+    if (nq > 0xFFFFFFFFu || !attn_rows_ok(S, (uint32_t)nq, hd) || groups > 0xFFFFFFFFu) return 0;
+    const uint32_t nch = rows_chunks(S, (uint32_t)groups);
+    return nch > 1 ? groups * nch * RQB * (hd + 2) : 0;
+}
+
+size_t attn_partial_floats(uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_kv, uint32_t hd) {
     const uint32_t nch = (S + ACH - 1) / ACH, cus = (uint32_t)device_cus();
     const size_t decode = (size_t)n_kv * nch * AQ * (AHD + 2);
     // k_attn_split: groups <= 4 n_kv (at most AQ queries per kv head), groups * chunks <= max(CUs, groups)
     const size_t gc = cus > 4 * n_kv ? cus : 4 * n_kv;
     const size_t split = gc * AQG * (AHD + 2) + (size_t)4 * n_kv * AQG;
-    return attn_cnt_floats(n_kv) + (decode > split ? decode : split);
+    // k_attn_rows: groups * chunks <= CUs, and no more chunks than rows_chunks' limits (the
+    // bound holds for fewer query heads too: a target's layers may differ in them)
+    const uint64_t groups = (uint64_t)n_kv * (((uint64_t)rows * (n_q / n_kv) + RQB - 1) / RQB);
+    const uint64_t cap = (S + RPT - 1) / RPT, wg = groups * (cap < 64 ? cap : 64);
+    const size_t many = hd == 64 || hd == AHD || hd == 256 ? (wg < cus ? wg : cus) * RQB * (hd + 2) : 0;
+    const size_t few = decode > split ? decode : split;
+    return attn_cnt_floats(n_kv) + (many > few ? many : few);
 }
 
-// `part` holds attn_partial_floats(S, n_kv) floats when the matrix-core path applies,
-// zeroed before its first use; `cnt` (when given) replaces its counters.  With `gate`
+template <int HD>
+int launch_attn_rows(RowsAttn &a, hipStream_t s) {
+    int dev = 0;
+    LG_HIP_TRY(hipGetDevice(&dev));
+    LG_REQUIRE(dev >= 0 && dev < 64, "attn_rows: device %d", dev);
+    static std::atomic<bool> lds_set[64];  // the kernel's LDS is past the 64 KiB default
+    if (!lds_set[dev].load(std::memory_order_acquire)) {
+        LG_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_attn_rows<HD>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(RowsLds<HD>)));
+        lds_set[dev].store(true, std::memory_order_release);
+    }
+    const uint64_t blocks = (uint64_t)(a.n_kv * a.nch + 7) / 8 * 8 * a.ngq;
+    hipLaunchKernelGGL(k_attn_rows<HD>, dim3((uint32_t)blocks), dim3(256), sizeof(RowsLds<HD>), s, a);
+    LG_TRY(after_launch("attn_rows", s));
+    if (a.nch == 1) return LG_OK;
+    hipLaunchKernelGGL(k_attn_rows_merge<HD>, dim3((a.rows * a.n_q + 3) / 4), dim3(256), 0, s, a);
+    return after_launch("attn_rows_merge", s);
+}
+
+// `part` holds attn_partial_floats(S, rows, n_q, n_kv, hd) floats when a matrix-core path
+// applies, zeroed before its first use (null: k_attn_rows with one chunk, or the plain kernel); `cnt` (when given) replaces its counters.  With `gate`
 // ([rows][n_q]) each head's result is multiplied by softplus of its gate.
 int run_attention(const float *q, const float *k0, const float *v0, uint32_t n0, const float *k1, const float *v1,
                   uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_kv, uint32_t hd, uint32_t qpos0, int causal,
@@ -1285,6 +1738,18 @@ int run_attention(const float *q, const float *k0, const float *v0, uint32_t n0,
         LG_TRY(run_qk_norm_rope(QkJob{}, QkJob{}, nullptr, hd, 0, 0.0f, s, *gj));
         gate = gj->out;
     }
+    const uint64_t ngq = ((uint64_t)rows * G + RQB - 1) / RQB;
+    if ((uint64_t)rows * n_q <= 0x7FFFFFFFu && attn_rows_ok(S, rows * G, hd) && al && aligned16_ptr(out) &&
+        ngq * n_kv <= 0x1000000u) {
+        RowsAttn a{};
+        a.q = q, a.k0 = k0, a.v0 = v0, a.k1 = k1, a.v1 = v1;
+        a.n0 = n0, a.S = S, a.rows = rows, a.n_q = n_q, a.n_kv = n_kv, a.qpos0 = qpos0, a.ngq = (uint32_t)ngq;
+        a.causal = causal, a.gmode = gmode, a.scale = scale, a.out = out, a.gate = gate;
+        a.nch = part ? rows_chunks(S, n_kv * a.ngq) : 1;
+        a.part_o = part ? part + attn_cnt_floats(n_kv) : nullptr;
+        a.part_ml = part ? a.part_o + (size_t)n_kv * a.ngq * a.nch * RQB * hd : nullptr;
+        return hd == 64 ? launch_attn_rows<64>(a, s) : hd == 256 ? launch_attn_rows<256>(a, s) : launch_attn_rows<AHD>(a, s);
+    }
     hipLaunchKernelGGL(k_attn_simple, dim3((rows * n_q + 3) / 4), dim3(256), 0, s, q, k0, v0, n0, k1, v1, S, rows,
                        n_q, n_kv, hd, qpos0, causal, scale, out);
     LG_TRY(after_launch("attn_simple", s));
@@ -1319,7 +1784,7 @@ uint64_t layout(const lg_dflash_hparams &hp, uint32_t m, uint32_t ctx_len, uint8
     const uint64_t ss_floats = (uint64_t)m * ((E + 63) / 64);  // at most one partial per 64 rows
     const uint64_t floats[] = {2 * m * E, 2 * m * E, 2 * m * KVD, 2 * m * KVD,  2 * m * QD, m * QD,
                                2 * (uint64_t)m * hp.n_heads,      m * E,        m * E,  m * FF, m * FF, m * A,
-                               attn_partial_floats(S, hp.n_kv_heads), (uint64_t)hp.n_layers * 2 * m * E,
+                               attn_partial_floats(S, m, hp.n_heads, hp.n_kv_heads, hp.head_dim), (uint64_t)hp.n_layers * 2 * m * E,
                                ss_floats, ss_floats, 2 * (uint64_t)m * 128};
     float **dst[] = {&L.xe, &L.nxe, &L.kk, &L.vv, &L.q, &L.att, &L.gate, &L.o, &L.h, &L.g, &L.u, &L.feat_n, &L.part,
                      &L.ny, &L.ssa, &L.ssb, &L.rope};
@@ -1786,7 +2251,9 @@ int glue_qk_norm_rope2(const float *q, const float *wq, float *q_out, uint32_t n
                             rope_dim, eps, s);
 }
 
-uint64_t glue_attn_partial_bytes(uint32_t seq_len, uint32_t n_kv) { return attn_partial_floats(seq_len, n_kv) * 4; }
+uint64_t glue_attn_partial_bytes(uint32_t seq_len, uint32_t n_q, uint32_t n_kv, uint32_t head_dim) {
+    return attn_partial_floats(seq_len, 1, n_q, n_kv, head_dim) * 4;
+}
 
 int glue_attention(const float *q, const float *k, const float *v, uint32_t seq_len, uint32_t q_pos, uint32_t n_q,
                    uint32_t n_kv, uint32_t head_dim, float *out, float *part, hipStream_t s, const float *gate) {
@@ -1908,9 +2375,19 @@ int lg_dispatch_mha_attn(const float *q, const float *k_seq, const float *v_seq,
     if (head_dim == AHD && rows * G <= AQ && seq_len) {
         void *p = nullptr;
         BufLease lease;
-        LG_TRY(stream_buffer(BUF_ATTN, s, attn_partial_floats(seq_len, n_kv_heads) * 4, lease, "lg_dispatch_mha_attn"));
+        LG_TRY(stream_buffer(BUF_ATTN, s, attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim) * 4, lease,
+                             "lg_dispatch_mha_attn"));
         p = lease.buf->ptr;
         part = static_cast<float *>(p);
+    } else if (rows_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim)) {
+        // k_attn_rows splits the sequence when there is a workspace for its partials, and
+        // takes it whole where none can be had (a capture before any such call)
+        BufLease lease;
+        if (stream_buffer(BUF_ATTN, s, attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim) * 4, lease,
+                          name) == LG_OK)
+            part = static_cast<float *>(lease.buf->ptr);
+        else
+            clear_error();
     }
     return run_attention(q, k_seq, v_seq, seq_len, nullptr, nullptr, seq_len, rows, n_q_heads, n_kv_heads, head_dim,
                          q_pos, causal, out, part, s);

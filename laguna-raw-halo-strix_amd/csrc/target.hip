@@ -37,7 +37,7 @@ uint64_t layout(const lg_target_model *md, uint32_t seq_len, uint8_t *base, TgtL
     const uint64_t E = hp.n_embd, H = max_q_dim(md), QD = H * hp.head_dim, KVD = (uint64_t)hp.n_kv_heads * hp.head_dim;
     const uint64_t FF = hp.n_ff;
     const uint64_t floats[] = {E, E, QD, KVD, KVD, QD, H, FF, FF, E, TABLE_FLOATS, TABLE_FLOATS,
-                               glue_attn_partial_bytes(seq_len, hp.n_kv_heads) / 4, E};
+                               glue_attn_partial_bytes(seq_len, (uint32_t)H, hp.n_kv_heads, hp.head_dim) / 4, E};
     float **dst[] = {&L.x, &L.nx, &L.q, &L.k, &L.v, &L.att, &L.gate, &L.g, &L.u, &L.o, &L.freq, &L.freq_swa, &L.part,
                      &L.x2};
     // the two RoPE tables first, at fixed offsets whatever seq_len is, so that an

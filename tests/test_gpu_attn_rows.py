@@ -1,0 +1,132 @@
+"""GPU: attention of many queries per kv head, and of head sizes 64 and 256, against the
+f64 oracle.  The kernel takes blocks of 64 queries over tiles of 32 positions, in one
+chunk or several, on f16 parts of its operands (1e-5 of the largest result, as the other
+matrix-core attention: measured below 2e-6); a tile that those parts cannot hold goes
+element by element."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import dflash_oracle as dfo
+import laguna_hip as lh
+import synth
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+def inputs(n_q, n_kv, hd, rows, S, seed):
+    return (synth.normal(seed, rows * n_q * hd).reshape(rows, -1), synth.normal(seed + 1, S * n_kv * hd).reshape(S, -1),
+            synth.normal(seed + 2, S * n_kv * hd).reshape(S, -1))
+
+
+def run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal=1):
+    qb, kb, vb = lh.upload_f32(ctx, q), lh.upload_f32(ctx, K), lh.upload_f32(ctx, V)
+    ob = lh.GpuBuffer(ctx, q.nbytes)
+    lh.dispatch_mha_attn_seq(ctx, qb, kb, vb, ob, n_q, n_kv, hd, K.shape[0], q_pos, rows=q.shape[0], causal=causal)
+    return ob.read_f32(q.size).reshape(q.shape)
+
+
+def check(y, want):
+    assert np.all(np.isfinite(y))
+    e = float(np.max(np.abs(y - want)) / np.max(np.abs(want)))
+    print(f"  |err|inf/|y|inf = {e:.2e}", flush=True)
+    assert e <= TOL
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S,q_pos,causal", [
+    (8, 2, 128, 17, 1, 0, 1),        # one position; 68 queries: a second block of four
+    (8, 8, 128, 65, 65, 0, 1),       # a whole causal triangle, one past a block and two tiles
+    (32, 8, 128, 32, 4095, 4063, 1),  # chunks merged, a ragged last tile
+    (4, 1, 128, 64, 96, 31, 0),      # not causal
+    (2, 2, 128, 130, 700, 600, 1),   # rows that see past the sequence's end
+    (4, 4, 64, 1, 33, 32, 1), (8, 2, 64, 20, 515, 400, 1),
+    (2, 1, 256, 1, 31, 30, 1), (8, 2, 256, 33, 300, 250, 1),
+    (64, 1, 128, 2, 200, 198, 1),    # 64 heads of one kv head
+])
+def test_attention_rows(ctx, n_q, n_kv, hd, rows, S, q_pos, causal):
+    print(f"attn n_q={n_q} n_kv={n_kv} hd={hd} rows={rows} S={S} q_pos={q_pos} causal={causal}", flush=True)
+    q, K, V = inputs(n_q, n_kv, hd, rows, S, 0x5EED0700 + S)
+    y = run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal)
+    check(y, dfo.attention(q, K, V, q_pos + np.arange(rows), n_q, n_kv, hd, causal=bool(causal)))
+    assert np.array_equal(y, run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal))
+
+
+@pytest.mark.parametrize("case", ["k_wide", "k_small", "q_wide", "v_wide", "v_small", "masked_nan", "v_inf", "k_ninf"])
+def test_attention_rows_range(ctx, case):
+    n_q, n_kv, hd, rows, S, q_pos = 32, 8, 128, 20, 300, 275
+    print(f"attn rows range: {case}", flush=True)
+    q, K, V = (a.reshape(a.shape[0], -1, hd) for a in inputs(n_q, n_kv, hd, rows, S, 0x5EED0720))
+    sees = np.ones((rows, n_q, hd), bool)
+    if case == "k_wide":  # a key far above f16's range against zero query elements
+        q[:, :, 5] = 0.0
+        K[37, 2, 5] = 7.0e30
+    elif case == "k_small":  # keys far below f16's, queries as far above
+        K *= np.float32(2.0 ** -60)
+        q *= np.float32(2.0 ** 60)
+    elif case == "q_wide":
+        K[:, :, 9] = 0.0
+        q[3, 9, 9] = 7.0e30
+    elif case == "v_wide":
+        V[100, 1, 17] = 7.0e30
+    elif case == "v_small":
+        V *= np.float32(2.0 ** -30)
+    elif case == "masked_nan":  # rows 0 .. 4 do not see position 280, no row sees 296 ..
+        V[280, 3, 7] = np.nan
+        K[296:], V[296:] = np.nan, np.inf
+        sees[5:, 12:16] = False  # the rows whose kv head 3 meets the NaN
+    elif case == "v_inf":
+        V[50, 0, 3] = np.inf
+        sees[:, :4, 3] = False
+    else:  # a key of -inf against positive queries: weight 0
+        q[:, :, 0] = np.abs(q[:, :, 0]) + 1.0
+        K[60, :, 0] = -np.inf
+    q, K, V = q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
+    y = run(ctx, q, K, V, n_q, n_kv, hd, q_pos).reshape(sees.shape)
+    ko, vo = K.copy(), V.copy()
+    ko[296:], vo[296:] = (0.0, 0.0) if case == "masked_nan" else (ko[296:], vo[296:])
+    with np.errstate(all="ignore"):
+        ko = np.where(np.isneginf(ko), -1e30, ko)
+        vo = np.where(np.isfinite(vo), vo, 0.0)
+        want = dfo.attention(q, ko, vo, q_pos + np.arange(rows), n_q, n_kv, hd).reshape(sees.shape)
+    check(y[sees], want[sees])
+    if case == "v_inf":
+        assert np.all(np.isposinf(y[~sees]))
+    if case == "masked_nan":  # element by element: only the NaN's own dim, in the rows that see it
+        assert np.all(np.isnan(y[5:, 12:16, 7])) and np.all(np.isfinite(np.delete(y, 7, axis=2)))
+
+
+def test_attention_rows_first_call_captured(ctx):
+    """A capture on a stream that has no workspace yet: the sequence is taken whole, and
+    the graph's result is the eager one's within rounding."""
+    n_q, n_kv, hd, rows, S = 32, 8, 128, 32, 1000
+    print("attn rows captured before any call on the stream", flush=True)
+    q, K, V = inputs(n_q, n_kv, hd, rows, S, 0x5EED0740)
+    hip = ctypes.CDLL("libamdhip64.so")
+    vp = ctypes.c_void_p
+    hip.hipStreamBeginCapture.argtypes = [vp, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [vp, ctypes.POINTER(vp)]
+    hip.hipGraphInstantiate.argtypes = [ctypes.POINTER(vp), vp, vp, vp, ctypes.c_size_t]
+    hip.hipGraphLaunch.argtypes, hip.hipGraphExecDestroy.argtypes, hip.hipGraphDestroy.argtypes = [vp, vp], [vp], [vp]
+    qb, kb, vb = lh.upload_f32(ctx, q), lh.upload_f32(ctx, K), lh.upload_f32(ctx, V)
+    ob = lh.GpuBuffer(ctx, q.nbytes)
+    run(ctx, q, K, V, n_q, n_kv, hd, S - rows)  # the kernel is loaded (on the null stream)
+    s, g, ge = lh.Stream(), vp(), vp()
+    assert hip.hipStreamBeginCapture(s.ptr, 1) == 0
+    st = lh.lib().lg_dispatch_mha_attn(qb.ptr, kb.ptr, vb.ptr, ob.ptr, n_q, n_kv, hd, S, S - rows, rows, 1, s.ptr)
+    assert hip.hipStreamEndCapture(s.ptr, ctypes.byref(g)) == 0
+    lh.check(st)
+    assert hip.hipGraphInstantiate(ctypes.byref(ge), g, None, None, 0) == 0
+    want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd)
+    for rep in range(3):
+        ob.fill(0xFF)
+        ctx.sync()
+        assert hip.hipGraphLaunch(ge, s.ptr) == 0
+        s.sync()
+        check(ob.read_f32(q.size).reshape(q.shape), want)
+        check(run(ctx, q, K, V, n_q, n_kv, hd, S - rows), want)
+    hip.hipGraphExecDestroy(ge)
+    hip.hipGraphDestroy(g)
+    s.destroy()
