@@ -189,6 +189,10 @@ uint64_t proj_batch_multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs,
 int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob *jobs, uint32_t njobs, uint32_t k,
                      uint32_t m, int w_dtype, void *ws, uint64_t ws_bytes, hipStream_t s, bool glu = false,
                      const RowScale *rs = nullptr, const QkRope *qk = nullptr);
+// The small-M product over f32 weights (1 <= m <= 64, k a multiple of 4, w and f32 x
+// 16-byte aligned, bf16 x 8-byte aligned): c = W x (+ res), no workspace.
+int proj_f32_mm(const void *x, bool x_bf16, const float *w, float *c, const float *res, uint32_t m, uint32_t k,
+                uint32_t n, hipStream_t s);
 uint32_t proj_batch_norm_cols(int w_dtype, uint32_t k, uint32_t n, uint32_t m);
 uint32_t proj_batch_rs_cols_max(uint32_t m);
 // Whether products with these weights (f32 activations, 16-byte aligned) take the

@@ -995,8 +995,8 @@ __global__ __launch_bounds__(256) void k_mm_mf(const void *x, const float *up, M
     mm_body<Q4, TT, RT, GLU, NORM, TILED, XM>(x, up, jobs, J_, cnt, m, k, row_bytes, ch, lrec, lstage);
 }
 
-// Fallback for shapes outside the MFMA path (f32 weights, k not a multiple of the
-// block, unaligned pointers, k = 0): one wavefront per output row, element-wise
+// Fallback for shapes outside the MFMA paths (k not a multiple of the block, or of 4 for f32
+// weights, unaligned pointers, f32 weights with up, k = 0): one wavefront per output row, element-wise
 // decode.  c = res + W x when res is given; x = silu(x) * up when up is given.
 __global__ __launch_bounds__(256) void k_generic_batch(const void *__restrict__ xv, int x_bf16,
                                                        const float *__restrict__ up, const void *__restrict__ wv,
@@ -1302,6 +1302,13 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
     if (!fast) {
         for (uint32_t j = 0; j < njobs; j++) {
             if (jb[j].n == 0) continue;
+            if (w_dtype == LG_F32 && k && k % 4 == 0 && !up &&
+                (reinterpret_cast<uintptr_t>(x) & (x_dtype == LG_F32 ? 15u : 7u)) == 0 &&
+                (reinterpret_cast<uintptr_t>(jb[j].w) & 15u) == 0) {
+                LG_TRY(proj_f32_mm(x, x_dtype == LG_BF16, static_cast<const float *>(jb[j].w), jb[j].c, jb[j].res, m, k,
+                                   jb[j].n, s));
+                continue;
+            }
             hipLaunchKernelGGL(k_generic_batch, dim3((jb[j].n + 3) / 4), dim3(256), 0, s, x, (int)(x_dtype == LG_BF16),
                                up, jb[j].w, jb[j].c, jb[j].res, m, k, jb[j].n, w_dtype);
             LG_TRY(after_launch(name, s));
