@@ -13,52 +13,57 @@ namespace {
 
 using namespace lg;
 
-// One thread per 16-byte quant chunk: 8 threads per 144-byte super-block, each
-// producing 32 values (16 low nibbles of sub-block 2g, 16 high nibbles of 2g+1).
+// Four consecutive values per thread, DQ_UNITS times: a wavefront's store is 1 KiB of
+// contiguous f32 (and, Q4_K, one super-block), whatever the format.  The stores are most
+// of the traffic (4 bytes against 0.56 to 2 read), so their layout sets the rate: with a
+// block of 32 or a 16-byte quant chunk per thread, its stores 64 or 128 bytes apart, 58.7 M
+// values took Q8_0 95 us and Q4_K 76.6, now 42.7 (7.0 TB/s) and 38.7; with ordinary instead
+// of nontemporal stores 65.2 and 51.5.
+constexpr uint32_t DQ_UNITS = 4, DQ_WG = DQ_UNITS * 1024;  // values per workgroup
+
+// Values e .. e + 3 (those below n) of out.
+__device__ __forceinline__ void dq_store(float *out, uint64_t e, uint64_t n, const float (&v)[4], int vec_out) {
+    if (vec_out && e + 4 <= n) {
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        __builtin_nontemporal_store((f32x4){v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4 *>(out + e));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (e + i < n) out[e + i] = v[i];
+    }
+}
+
 __global__ __launch_bounds__(256) void k_dequant_q4k(const uint8_t *__restrict__ data,
                                                      uint64_t blocks_avail, uint64_t n,
                                                      float *__restrict__ out, int vec_out) {
-    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t b = gid >> 3;
-    const uint32_t c = gid & 7u, g = c >> 1, h = c & 1u;
-    const uint64_t base = b * QK_K + 64u * g + 16u * h;  // first low-nibble element
-    if (base >= n) return;
-    float lo[16], hi[16];
-    if (b < blocks_avail) {
-        const uint8_t *blk = data + b * Q4K_BYTES;
-        const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-        const uint4 qs = *reinterpret_cast<const uint4 *>(blk + 16 + 32 * g + 16 * h);
-        const float d = ref_half(hd.x & 0xFFFFu), dmin = ref_half(hd.x >> 16);
-        uint32_t sc0, m0, sc1, m1;
-        scale_min_k4(2 * g, hd.y, hd.z, hd.w, sc0, m0);
-        scale_min_k4(2 * g + 1, hd.y, hd.z, hd.w, sc1, m1);
-        const float a0 = __fmul_rn(d, (float)sc0), b0 = __fmul_rn(dmin, (float)m0);
-        const float a1 = __fmul_rn(d, (float)sc1), b1 = __fmul_rn(dmin, (float)m1);
-        const uint32_t w[4] = {qs.x, qs.y, qs.z, qs.w};
+    const uint64_t e0 = (uint64_t)blockIdx.x * DQ_WG + 4u * threadIdx.x;
+    const uint32_t w = 4u * (threadIdx.x & 63u), g = w >> 6, hi = (w >> 5) & 1u;  // this thread's place in its super-block
+    uint4 hd[DQ_UNITS];
+    uint32_t qs[DQ_UNITS];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint32_t byte = (w[i >> 2] >> (8 * (i & 3))) & 0xFFu;
-            lo[i] = __fsub_rn(__fmul_rn(a0, (float)(byte & 15u)), b0);
-            hi[i] = __fsub_rn(__fmul_rn(a1, (float)(byte >> 4)), b1);
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t b = (e0 + 1024u * u) / QK_K;
+        if (b < blocks_avail) {
+            const uint8_t *blk = data + b * Q4K_BYTES;
+            hd[u] = *reinterpret_cast<const uint4 *>(blk);
+            qs[u] = *reinterpret_cast<const uint32_t *>(blk + 16 + 32 * g + (w & 31u));
         }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; i++) lo[i] = hi[i] = 0.0f;
     }
-    if (vec_out && base + 48 <= n) {
-        float4 *o = reinterpret_cast<float4 *>(out + base);
-        float4 *p = reinterpret_cast<float4 *>(out + base + 32);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            o[i] = make_float4(lo[4 * i], lo[4 * i + 1], lo[4 * i + 2], lo[4 * i + 3]);
-            p[i] = make_float4(hi[4 * i], hi[4 * i + 1], hi[4 * i + 2], hi[4 * i + 3]);
-        }
-    } else {
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t e = e0 + 1024u * u, b = e / QK_K;
+        if (e >= n) break;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (b < blocks_avail) {
+            uint32_t sc, mn;
+            scale_min_k4(2 * g + hi, hd[u].y, hd[u].z, hd[u].w, sc, mn);
+            const float a = __fmul_rn(ref_half(hd[u].x & 0xFFFFu), (float)sc);
+            const float c = __fmul_rn(ref_half(hd[u].x >> 16), (float)mn);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            if (base + i < n) out[base + i] = lo[i];
-            if (base + 32 + i < n) out[base + 32 + i] = hi[i];
+            for (int i = 0; i < 4; i++)
+                v[i] = __fsub_rn(__fmul_rn(a, (float)((qs[u] >> (8 * i + 4 * hi)) & 15u)), c);
         }
+        dq_store(out, e, n, v, vec_out);
     }
 }
 
@@ -86,35 +91,56 @@ __global__ __launch_bounds__(256) void k_dequant_q4k_bytes(const uint8_t *__rest
     out[i] = __fsub_rn(__fmul_rn(__fmul_rn(d, (float)sc), q), __fmul_rn(dmin, (float)mn));
 }
 
-// One thread per 34-byte Q8_0 block (value = float(q) * d, src/dflash.rs:389-394).
+// value = float(q) * d (src/dflash.rs:389-394).  A2: the tensor's base is 2-byte aligned
+// (blocks of 34 bytes keep that).
+template <bool A2>
+__device__ __forceinline__ uint32_t dq_u16(const uint8_t *p) {
+    if constexpr (A2) return *reinterpret_cast<const uint16_t *>(p);
+    else return p[0] | (p[1] << 8);
+}
+
+template <bool A2>
 __global__ __launch_bounds__(256) void k_dequant_q8_0(const uint8_t *__restrict__ data,
                                                       uint64_t blocks_avail, uint64_t n,
                                                       float *__restrict__ out, int vec_out) {
-    const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t base = b * QK8_0;
-    if (base >= n) return;
-    float v[32];
-    if (b < blocks_avail) {
-        const uint8_t *blk = data + b * Q80_BYTES;
-        const float d = ref_half(blk[0] | (blk[1] << 8));
+    const uint64_t e0 = (uint64_t)blockIdx.x * DQ_WG + 4u * threadIdx.x;
+    uint32_t d[DQ_UNITS], q[DQ_UNITS];
 #pragma unroll
-        for (int i = 0; i < 32; i++) v[i] = __fmul_rn((float)(int8_t)blk[2 + i], d);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 32; i++) v[i] = 0.0f;
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t e = e0 + 1024u * u, b = e / QK8_0;
+        d[u] = q[u] = 0u;
+        if (b < blocks_avail) {
+            const uint8_t *blk = data + b * Q80_BYTES, *p = blk + 2 + e % QK8_0;
+            d[u] = dq_u16<A2>(blk);
+            q[u] = dq_u16<A2>(p) | (dq_u16<A2>(p + 2) << 16);
+        }
     }
-    if (vec_out && base + 32 <= n) {
-        float4 *o = reinterpret_cast<float4 *>(out + base);
 #pragma unroll
-        for (int i = 0; i < 8; i++) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    } else {
-        for (int i = 0; i < 32; i++)
-            if (base + i < n) out[base + i] = v[i];
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t e = e0 + 1024u * u;
+        if (e >= n) break;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (e / QK8_0 < blocks_avail) {
+            const float df = ref_half(d[u]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __fmul_rn((float)(int8_t)(q[u] >> (8 * i)), df);
+        }
+        dq_store(out, e, n, v, vec_out);
     }
 }
 
-// F32 / F16 / "BF16" branches (src/dflash.rs:333-378, :437-462), element-wise,
-// with the reference's per-element length check.
+// F32 / F16 / "BF16" branches (src/dflash.rs:333-378, :437-462), with the reference's
+// per-element length check.
+__device__ __forceinline__ float dq_half(uint32_t h, bool bf16) {
+    if (bf16) return ref_half(h);
+    // LG_F16: IEEE subnormals, canonical NaN
+    const uint32_t e = (h >> 10) & 31u, m = h & 0x3FFu;
+    const float sign = (h & 0x8000u) ? -1.0f : 1.0f;
+    if (e == 0) return __fmul_rn(__fmul_rn(sign, 6.103515625e-05f), __fdiv_rn((float)m, 1024.0f));
+    if (e == 31) return m == 0 ? sign * __builtin_inff() : __uint_as_float(0x7FC00000u);
+    return __fmul_rn(__fmul_rn(sign, ldexpf(1.0f, (int)e - 15)), __fadd_rn(1.0f, __fdiv_rn((float)m, 1024.0f)));
+}
+
 __global__ __launch_bounds__(256) void k_dequant_elem(const uint8_t *__restrict__ data, uint64_t len,
                                                       int dtype, uint64_t n, float *__restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -125,21 +151,57 @@ __global__ __launch_bounds__(256) void k_dequant_elem(const uint8_t *__restrict_
             r = __uint_as_float(data[4 * i] | (data[4 * i + 1] << 8) | (data[4 * i + 2] << 16) |
                                 ((uint32_t)data[4 * i + 3] << 24));
     } else if (i * 2 + 2 <= len) {
-        const uint32_t h = data[2 * i] | (data[2 * i + 1] << 8);
-        if (dtype == LG_BF16) {
-            r = ref_half(h);
-        } else {  // LG_F16: IEEE subnormals, canonical NaN
-            const uint32_t e = (h >> 10) & 31u, m = h & 0x3FFu;
-            const float sign = (h & 0x8000u) ? -1.0f : 1.0f;
-            if (e == 0) r = __fmul_rn(__fmul_rn(sign, 6.103515625e-05f), __fdiv_rn((float)m, 1024.0f));
-            else if (e == 31) r = m == 0 ? sign * __builtin_inff() : __uint_as_float(0x7FC00000u);
-            else r = __fmul_rn(__fmul_rn(sign, ldexpf(1.0f, (int)e - 15)), __fadd_rn(1.0f, __fdiv_rn((float)m, 1024.0f)));
-        }
+        r = dq_half(data[2 * i] | (data[2 * i + 1] << 8), dtype == LG_BF16);
     }
     out[i] = r;
 }
 
+// The same over a whole, 16-byte aligned tensor (len covers all n elements), four values a
+// load.  F16 codes other than NaNs decode as the hardware conversion does (exact).
+__global__ __launch_bounds__(256) void k_dequant_elem4(const uint8_t *__restrict__ data, int dtype, uint64_t n,
+                                                       float *__restrict__ out, int vec_out) {
+    const uint64_t e0 = (uint64_t)blockIdx.x * DQ_WG + 4u * threadIdx.x;
+    uint4 w[DQ_UNITS];
+#pragma unroll
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t e = e0 + 1024u * u;
+        if (e + 4 <= n) {
+            if (dtype == LG_F32) {
+                w[u] = *reinterpret_cast<const uint4 *>(data + 4 * e);
+            } else {
+                const uint2 h = *reinterpret_cast<const uint2 *>(data + 2 * e);
+                w[u] = make_uint4(h.x & 0xFFFFu, h.x >> 16, h.y & 0xFFFFu, h.y >> 16);
+            }
+        } else {  // the last one to three values
+            uint32_t t[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (e + i < n)
+                    t[i] = dtype == LG_F32 ? reinterpret_cast<const uint32_t *>(data)[e + i]
+                                           : reinterpret_cast<const uint16_t *>(data)[e + i];
+            w[u] = make_uint4(t[0], t[1], t[2], t[3]);
+        }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < DQ_UNITS; u++) {
+        const uint64_t e = e0 + 1024u * u;
+        if (e >= n) break;
+        const uint32_t t[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (dtype == LG_F32) v[i] = __uint_as_float(t[i]);
+            else if (dtype == LG_BF16) v[i] = ref_half(t[i]);
+            else
+                v[i] = (t[i] & 0x7FFFu) > 0x7C00u ? __uint_as_float(0x7FC00000u)
+                                                  : (float)__builtin_bit_cast(_Float16, (uint16_t)t[i]);
+        }
+        dq_store(out, e, n, v, vec_out);
+    }
+}
+
 inline unsigned grid_for(uint64_t threads) { return (unsigned)((threads + 255) / 256); }
+inline unsigned dq_grid(uint64_t n) { return (unsigned)((n + DQ_WG - 1) / DQ_WG); }
 
 }  // namespace
 
@@ -161,7 +223,7 @@ extern "C" int lg_dequant_to_f32(const void *data, uint64_t data_len, int dtype,
         const uint64_t need = (n + QK_K - 1) / QK_K, have = data_len / Q4K_BYTES;
         const uint64_t avail = have < need ? have : need;
         if ((reinterpret_cast<uintptr_t>(d) & 15u) == 0)
-            hipLaunchKernelGGL(k_dequant_q4k, dim3(grid_for(need * 8)), dim3(256), 0, s, d, avail, n, out, vec_out);
+            hipLaunchKernelGGL(k_dequant_q4k, dim3(dq_grid(n)), dim3(256), 0, s, d, avail, n, out, vec_out);
         else
             hipLaunchKernelGGL(k_dequant_q4k_bytes, dim3(grid_for(n)), dim3(256), 0, s, d, avail, n, out);
         return after_launch("dequant_q4k", s);
@@ -169,12 +231,19 @@ extern "C" int lg_dequant_to_f32(const void *data, uint64_t data_len, int dtype,
     case LG_Q8_0: {
         const uint64_t need = (n + QK8_0 - 1) / QK8_0, have = data_len / Q80_BYTES;
         const uint64_t avail = have < need ? have : need;
-        hipLaunchKernelGGL(k_dequant_q8_0, dim3(grid_for(need)), dim3(256), 0, s, d, avail, n, out, vec_out);
+        if ((reinterpret_cast<uintptr_t>(d) & 1u) == 0)
+            hipLaunchKernelGGL(k_dequant_q8_0<true>, dim3(dq_grid(n)), dim3(256), 0, s, d, avail, n, out, vec_out);
+        else
+            hipLaunchKernelGGL(k_dequant_q8_0<false>, dim3(dq_grid(n)), dim3(256), 0, s, d, avail, n, out, vec_out);
         return after_launch("dequant_q8_0", s);
     }
     case LG_F32:
     case LG_F16:
     case LG_BF16:
+        if ((reinterpret_cast<uintptr_t>(d) & 15u) == 0 && data_len / (dtype == LG_F32 ? 4 : 2) >= n) {
+            hipLaunchKernelGGL(k_dequant_elem4, dim3(dq_grid(n)), dim3(256), 0, s, d, dtype, n, out, vec_out);
+            return after_launch("dequant_elem", s);
+        }
         hipLaunchKernelGGL(k_dequant_elem, dim3(grid_for(n)), dim3(256), 0, s, d, data_len, dtype, n, out);
         return after_launch("dequant_elem", s);
     default:  // src/dflash.rs:463: unsupported types decode to zeros
