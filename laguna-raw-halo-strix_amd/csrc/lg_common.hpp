@@ -189,6 +189,10 @@ uint64_t proj_batch_multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs,
 int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob *jobs, uint32_t njobs, uint32_t k,
                      uint32_t m, int w_dtype, void *ws, uint64_t ws_bytes, hipStream_t s, bool glu = false,
                      const RowScale *rs = nullptr, const QkRope *qk = nullptr);
+// M = 1 over raw Q8_0 rows of whole blocks (k a multiple of 32; up: silu(x) * up), and
+// whether a call's sizes and alignment qualify.
+bool proj_q80_rows_ok(uint32_t k, uint32_t n, const float *x, const float *up, const void *w);
+int proj_q80_rows(const float *x, const float *up, const void *w, float *y, uint32_t k, uint32_t n, hipStream_t s);
 // The small-M product over f32 weights (1 <= m <= 64, k a multiple of 4, w and f32 x
 // 16-byte aligned, bf16 x 8-byte aligned): c = W x (+ res), no workspace.
 int proj_f32_mm(const void *x, bool x_bf16, const float *w, float *c, const float *res, uint32_t m, uint32_t k,

@@ -28,8 +28,9 @@
 //    the last workgroup to finish.
 //
 // Q8_0 with k <= 4096: integer dot products against activation digits (k_q80_m1_dig,
-// described there).  Q8_0 with k > 4096: vector ALU.  A "team" of TW = min(4, ceil(k/4096)) waves covers one row (in
-// passes of 16384 elements beyond that): lane p of
+// described there).  Q8_0 with k > 4096, the fused path over Q8_0 and k no multiple of 256:
+// proj_q80_rows, up to its longest row.  Plain Q8_0 beyond that: vector ALU (k_q80_m1).  A
+// "team" of TW waves covers one row in passes of 4096 TW elements: lane p of
 // the team owns the 64-element group p of the row (two 34-byte blocks, 68 bytes,
 // dword aligned) and keeps the 64 activations of that group in registers; the
 // team's partial sums meet in a DPP/swizzle wavefront reduction (plus LDS across
@@ -1863,9 +1864,7 @@ int launch_q80(const float *x, const uint8_t *w, float *y, uint32_t k, uint32_t 
                            (uint64_t)k / QK8_0 * Q80_BYTES);
         return after_launch("proj_q8_0_m1", s);
     }
-    if (P <= 128) return launch_q80_t<2, 4>(x, w, y, k, n, s);
-    if (P <= 192) return launch_q80_t<3, 2>(x, w, y, k, n, s);
-    return launch_q80_t<4, 2>(x, w, y, k, n, s);
+    return launch_q80_t<4, 2>(x, w, y, k, n, s);  // past proj_q80_rows' longest row
 }
 
 // Shared front end of every quantized M=1 entry point.
@@ -1912,7 +1911,12 @@ int proj_quant(const float *x, const float *up, const void *w, float *c, uint32_
                         : launch_q4k_mfma<true>(x, up, wbase, c, k, n, s);
         }
     }
-    if (dtype == LG_Q8_0 && vec_ok && !fuse && aligned16(wb)) return launch_q80(x, wb, c, k, n, s);
+    if (dtype == LG_Q8_0) {
+        const bool q80 = vec_ok && !fuse && aligned16(wb);
+        if (q80 && k <= 4096) return launch_q80(x, wb, c, k, n, s);
+        if (proj_q80_rows_ok(k, n, x, up, wb)) return proj_q80_rows(x, up, wb, c, k, n, s);
+        if (q80) return launch_q80(x, wb, c, k, n, s);
+    }
     if (dtype == LG_F32 && !fuse) {
         hipLaunchKernelGGL(k_f32_rows, dim3((n + 3) / 4), dim3(256), 0, s, x, reinterpret_cast<const float *>(w), c, k,
                            n, (int)(aligned16(x) && aligned16(w) && k % 4 == 0));
