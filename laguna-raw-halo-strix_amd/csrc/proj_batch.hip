@@ -65,16 +65,24 @@ __device__ __forceinline__ f16x8 as_f16x8(uint32_t a, uint32_t b, uint32_t c, ui
     return __builtin_bit_cast(f16x8, make_uint4(a, b, c, d));
 }
 
-// Fragment record of one (16-token tile, 256-element chunk) in LDS, FR_U4 16-byte words:
+// Fragment record of one (16-token tile, 256-element chunk) in LDS, Fr<NP>::U4 16-byte words:
 //   [0, 1024)     word (j*2 + p)*64 + (l ^ (2j + l/32)): part p (0 = hi, 1 = lo) of
 //                 sub-block j's A operand, lane l: token l%16, elements
 //                 32j + 8(l/16) + {0,2,1,3,4,6,5,7}.  The XOR spreads over all LDS banks
 //                 the 16 threads of one token that store a word together (thread q of
 //                 the token stores lane slots 16(2(q%2) + h) + token, XOR q)
+//   (bf16 activations: hi alone, lo is 0 -- 8 significant bits lie in hi, and what hi's
+//   subnormal step drops lies below lo's; words j*64 + ..., and the rest 512 words earlier;
+//   half the matrix products: with the wide launches Q4_K 4096 -> 14336 at m = 40 50.1 ->
+//   28.6 us)
 //   [1024, 1056)  float2 per lane l: (X[l%16][l/16], X[l%16][l/16 + 4]), X the sums of
 //                 the scaled values over each sub-block
 //   [1056, 1060)  the 16 tokens' 2^-e
-constexpr uint32_t FR_X = 1024, FR_S = 1056, FR_U4 = 1060;
+// NP: parts (2, or 1 for bf16).
+template <int NP>
+struct Fr {
+    static constexpr uint32_t X = 512 * NP, S = X + 32, U4 = X + 36;
+};
 
 // 2^-24 scaled codes: Q4_K nibbles in place (low nibbles of bytes 0 and 2 / 1 and 3
 // of a dword: `& LO4`, high nibbles `& HI4`), Q8_0 bytes biased to unsigned.
@@ -96,7 +104,16 @@ constexpr uint32_t LO4 = 0x000F000Fu, HI4 = 0x00F000F0u, LO8 = 0x00FF00FFu;
 //    The workgroup that finishes a column computes the scales, with the slices'
 //    partial sums in flight.
 constexpr int MM_JOBS = 4;
-constexpr uint32_t MM_SS_LOADS = 8;  // partial sums a consuming lane loads (per-token capacity 8 * 16 / TT)
+// Lanes per token of a consuming workgroup (its 256 threads over TT tiles of 16 tokens, 3
+// as 4), and the partial sums each loads: a capacity of 128 per token for one tile, else 64.
+template <int TT>
+constexpr uint32_t mm_lt() {
+    return 16 / (TT == 3 ? 4 : TT);
+}
+template <int TT>
+constexpr uint32_t mm_ss_loads() {
+    return TT > 2 ? 16 : 8;
+}
 struct MmJob {
     const uint8_t *w;
     float *out;
@@ -107,7 +124,7 @@ struct MmJob {
     float *ss;
     uint32_t n, g0;
     const float *qkw;  // QK-norm weights (heads of 128 rows, RT = 2), or null
-    uint32_t tlo;      // 1: only the second token tile of a two-tile launch is needed
+    uint32_t tlo;      // 1: the first token tile of two, or the first two of three or four, are not needed
 };
 struct MmJobs {
     MmJob j[MM_JOBS];
@@ -151,17 +168,17 @@ __device__ __forceinline__ float row16_max(float v) {
 }
 
 
-// NORM: token threadIdx.x / LT of the launch (LT = 16 / TT lanes per token) takes its
+// NORM: token threadIdx.x / LT of the launch (LT lanes per token) takes its
 // partial sums p = sub, sub + LT, ... (branch-free: slots past the columns and tokens
 // without a scale read a valid slot, dropped in rs_store).
 template <int TT>
-__device__ __forceinline__ void ss_load(float (&ssv)[MM_SS_LOADS], const MmJobs &jobs, uint32_t m) {
-    constexpr uint32_t LT = 16 / TT;
+__device__ __forceinline__ void ss_load(float (&ssv)[mm_ss_loads<TT>()], const MmJobs &jobs, uint32_t m) {
+    constexpr uint32_t LT = mm_lt<TT>();
     const uint32_t tok = threadIdx.x / LT, sub = threadIdx.x % LT, cols = jobs.rs_cols, tok0 = jobs.rs_tok0;
     const uint32_t rows = m > tok0 ? m - tok0 : 1u;
     const uint32_t r = tok >= tok0 && tok - tok0 < rows ? tok - tok0 : 0u;
 #pragma unroll
-    for (uint32_t j = 0; j < MM_SS_LOADS; j++) {
+    for (uint32_t j = 0; j < mm_ss_loads<TT>(); j++) {
         const uint32_t p = sub + LT * j;
         ssv[j] = jobs.rs_ss[(uint64_t)r * cols + (p < cols ? p : cols - 1)];
     }
@@ -169,23 +186,24 @@ __device__ __forceinline__ void ss_load(float (&ssv)[MM_SS_LOADS], const MmJobs 
 
 // NORM: rsl[t] = (sum of token t's partials / k + eps)^-1/2, or 1 for tokens below
 // tok0 (and past m).  The lanes of a token add their slots in slot order, then meet
-// in DPP steps within their 16-lane row: xor 1, xor 2 (quad_perm), the half-row
-// mirror (lane i and 7 - i of each 8) and, for 16 lanes per token, the row mirror
+// in DPP steps within their 16-lane row: xor 1, xor 2 (quad_perm), from 8 lanes per token
+// the half-row mirror (lane i and 7 - i of each 8) and, for 16, the row mirror
 // (i and 15 - i).  Every lane of the token ends with the sum.
 template <int TT>
-__device__ __forceinline__ void rs_store(const float (&ssv)[MM_SS_LOADS], float *rsl, const MmJobs &jobs, uint32_t m,
+__device__ __forceinline__ void rs_store(const float (&ssv)[mm_ss_loads<TT>()], float *rsl, const MmJobs &jobs, uint32_t m,
                                          uint32_t k) {
-    constexpr uint32_t LT = 16 / TT;
+    constexpr uint32_t LT = mm_lt<TT>();
     const uint32_t tok = threadIdx.x / LT, sub = threadIdx.x % LT, tok0 = jobs.rs_tok0;
     float s = 0.0f;
 #pragma unroll
-    for (uint32_t j = 0; j < MM_SS_LOADS; j++) s += sub + LT * j < jobs.rs_cols ? ssv[j] : 0.0f;
+    for (uint32_t j = 0; j < mm_ss_loads<TT>(); j++) s += sub + LT * j < jobs.rs_cols ? ssv[j] : 0.0f;
     s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
     s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x141, 0xF, 0xF, false));  // row_half_mirror
+    if constexpr (LT >= 8)
+        s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x141, 0xF, 0xF, false));  // row_half_mirror
     if constexpr (LT == 16)
         s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x140, 0xF, 0xF, false));  // row_mirror
-    if (sub == 0) rsl[tok] = tok >= tok0 && tok < m ? 1.0f / sqrtf(s / (float)k + jobs.rs_eps) : 1.0f;
+    if (sub == 0 && tok < TT * 16) rsl[tok] = tok >= tok0 && tok < m ? 1.0f / sqrtf(s / (float)k + jobs.rs_eps) : 1.0f;
 }
 
 // The workgroup's results: the output itself (one slice), or its slice's partial
@@ -280,7 +298,7 @@ __device__ __forceinline__ void finish(const float (&acc)[RT][TT][4], float *out
     }
     // NORM: the partial sums of squares behind the token scales, loaded with the
     // slices' partial sums (only the workgroup that finishes a column reads them)
-    float ssv[MM_SS_LOADS];
+    float ssv[mm_ss_loads<TT>()];
     if constexpr (NORM) ss_load<TT>(ssv, jobs, m);
     // Slices are added in slice order (the sum does not depend on arrival order);
     // the loads of G slices for all RT row tiles are in flight together.
@@ -607,8 +625,10 @@ __device__ __forceinline__ void stage_q4k(const Q4kRawChunk<RT> &R, Q4kChunk<RT>
 // never stored).
 template <int TT, int XM>
 struct RecBuild {
-    float v[TT][16];
+    static constexpr int NP = XM == 1 ? 1 : 2;
+    float v[XM == 1 ? 1 : TT][16];
     float u[XM == 2 ? TT : 1][16];
+    lg_u32x4 h[XM == 1 ? TT : 1][2];  // bf16: kept as loaded until the record is built
     __device__ __forceinline__ void load(const void *x, const float *up, uint32_t m, uint32_t k, uint32_t c) {
         const uint32_t tok = threadIdx.x >> 4, q = threadIdx.x & 15u;
 #pragma unroll
@@ -616,14 +636,9 @@ struct RecBuild {
             const uint32_t tr = t * 16 + tok;
             const uint64_t e0 = (uint64_t)(tr < m ? tr : m - 1) * k + (uint64_t)QK_K * c + 16 * q;
             if constexpr (XM == 1) {
-                const uint4 *p = reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(x) + e0);
-                const uint4 h0 = p[0], h1 = p[1];
-                const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    v[t][2 * i] = bf16_to_f32(hw[i] & 0xFFFFu);
-                    v[t][2 * i + 1] = __uint_as_float(hw[i] & 0xFFFF0000u);
-                }
+                const lg_u32x4 *p = reinterpret_cast<const lg_u32x4 *>(static_cast<const uint16_t *>(x) + e0);
+                h[t][0] = p[0];
+                h[t][1] = p[1];
             } else {
                 const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(x) + e0);
 #pragma unroll
@@ -655,11 +670,16 @@ struct RecBuild {
             float w[16], amax = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                float a = v[t][i];
-                if constexpr (XM == 2) a = silu_mul(a, u[t][i]);  // kernels/activation.comp:21-28
-                w[i] = a;
-                amax = fmaxf(amax, fabsf(w[i]));
+                if constexpr (XM == 1) {
+                    const uint32_t hw = h[t][i >> 3][(i >> 1) & 3];
+                    w[i] = __uint_as_float(i & 1 ? hw & 0xFFFF0000u : hw << 16);
+                } else {
+                    w[i] = v[t][i];
+                }
+                if constexpr (XM == 2) w[i] = silu_mul(w[i], u[t][i]);  // kernels/activation.comp:21-28
             }
+#pragma unroll
+            for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(w[i]));
             amax = row16_max(amax);
             // 2^e puts the chunk's largest magnitude in [2^14, 2^15); a zero or non-finite
             // chunk keeps e = 0 (non-finite values then reach the products as f16 inf / NaN)
@@ -675,57 +695,60 @@ struct RecBuild {
                 sum += sv[i];
             }
             // the two f16 parts of elements i, i + 2 in one word each (v_cvt_pk_f16_f32,
-            // round to nearest even): hi the nearest f16, lo that of the exact remainder
+            // round to nearest even): hi the nearest f16, lo that of the exact remainder.
+            // (v_fma_mixlo / mixhi_f16 give both parts and the scaling in two instructions an
+            // element instead of three, and measured slower: the draft block 572 -> 581 us)
             uint32_t hp[8], lp[8];
 #pragma unroll
             for (int c = 0; c < 8; c++) {
                 const int i0 = 8 * (c >> 2) + (c & 1) + 4 * ((c >> 1) & 1), i1 = i0 + 2;
                 const f16x2_t hv = __builtin_convertvector((f32x2_t){sv[i0], sv[i1]}, f16x2_t);
-                const uint32_t hw = __builtin_bit_cast(uint32_t, hv);
-                // sv - hi, exact, straight from the packed f16 halves (one v_fma_mix_f32 each)
-                float r0, r1;
-                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hw), "v"(sv[i0]));
-                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hw), "v"(sv[i1]));
-                const f16x2_t lv = __builtin_convertvector((f32x2_t){r0, r1}, f16x2_t);
-                hp[c] = hw;
-                lp[c] = __builtin_bit_cast(uint32_t, lv);
+                hp[c] = __builtin_bit_cast(uint32_t, hv);
+                if constexpr (NP == 2) {
+                    // sv - hi, exact, straight from the packed f16 halves (one v_fma_mix_f32 each)
+                    float r0, r1;
+                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hp[c]), "v"(sv[i0]));
+                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hp[c]), "v"(sv[i1]));
+                    lp[c] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){r0, r1}, f16x2_t));
+                }
             }
             // the sub-block's sum: this thread's 16 and its neighbour's (q ^ 1), the same
             // float in both (addition is commutative)
             sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xB1, 0xF, 0xF, false));
-            uint4 *rec = lds + t * FR_U4;
+            uint4 *rec = lds + t * Fr<NP>::U4;
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint32_t lane = ((q & 1u) * 2 + h) * 16 + tok;
-                rec[(j * 2 + 0) * 64 + (lane ^ q)] = make_uint4(hp[4 * h], hp[4 * h + 1], hp[4 * h + 2], hp[4 * h + 3]);
-                rec[(j * 2 + 1) * 64 + (lane ^ q)] = make_uint4(lp[4 * h], lp[4 * h + 1], lp[4 * h + 2], lp[4 * h + 3]);
+            for (int h2 = 0; h2 < 2; h2++) {
+                const uint32_t lane = ((q & 1u) * 2 + h2) * 16 + tok;
+                rec[(j * NP + 0) * 64 + (lane ^ q)] = make_uint4(hp[4 * h2], hp[4 * h2 + 1], hp[4 * h2 + 2], hp[4 * h2 + 3]);
+                if constexpr (NP == 2)
+                    rec[(j * 2 + 1) * 64 + (lane ^ q)] = make_uint4(lp[4 * h2], lp[4 * h2 + 1], lp[4 * h2 + 2], lp[4 * h2 + 3]);
             }
             float *rf = reinterpret_cast<float *>(rec);
-            if ((q & 1u) == 0) rf[4 * FR_X + ((j & 3u) * 16 + tok) * 2 + (j >> 2)] = sum;
-            if (q == 0) rf[4 * FR_S + tok] = __builtin_ldexpf(1.0f, -e);
+            if ((q & 1u) == 0) rf[4 * Fr<NP>::X + ((j & 3u) * 16 + tok) * 2 + (j >> 2)] = sum;
+            if (q == 0) rf[4 * Fr<NP>::S + tok] = __builtin_ldexpf(1.0f, -e);
         }
     }
 };
 
 // The chunk's min / bias terms and token scales: tmp += X (16x4) * coef (4x16) for
 // sub-blocks kg and kg + 4, then acc += tmp * 2^-e per token.
-template <int TT, int RT>
+template <int NP, int TT, int RT, int TA>
 __device__ __forceinline__ void chunk_close(const uint4 *lds, f32x4 (&tmp)[RT][TT], const float (&cm)[RT][2],
-                                            float (&acc)[RT][TT][4]) {
+                                            float (&acc)[RT][TA][4], int ta) {
     const uint32_t l = threadIdx.x & 63u, kg = l >> 4;
 #pragma unroll
     for (int t = 0; t < TT; t++) {
-        const float2 xv = reinterpret_cast<const float2 *>(lds + t * FR_U4 + FR_X)[l];
-        const float4 sv = reinterpret_cast<const float4 *>(lds + t * FR_U4 + FR_S)[kg];
+        const float2 xv = reinterpret_cast<const float2 *>(lds + t * Fr<NP>::U4 + Fr<NP>::X)[l];
+        const float4 sv = reinterpret_cast<const float4 *>(lds + t * Fr<NP>::U4 + Fr<NP>::S)[kg];
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             f32x4 C = tmp[i][t];
             C = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.x, cm[i][0], C, 0, 0, 0);
             C = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.y, cm[i][1], C, 0, 0, 0);
-            acc[i][t][0] = __builtin_fmaf(C[0], sv.x, acc[i][t][0]);
-            acc[i][t][1] = __builtin_fmaf(C[1], sv.y, acc[i][t][1]);
-            acc[i][t][2] = __builtin_fmaf(C[2], sv.z, acc[i][t][2]);
-            acc[i][t][3] = __builtin_fmaf(C[3], sv.w, acc[i][t][3]);
+            acc[i][ta + t][0] = __builtin_fmaf(C[0], sv.x, acc[i][ta + t][0]);
+            acc[i][ta + t][1] = __builtin_fmaf(C[1], sv.y, acc[i][ta + t][1]);
+            acc[i][ta + t][2] = __builtin_fmaf(C[2], sv.z, acc[i][ta + t][2]);
+            acc[i][ta + t][3] = __builtin_fmaf(C[3], sv.w, acc[i][ta + t][3]);
         }
     }
 }
@@ -735,8 +758,8 @@ __device__ __forceinline__ void chunk_close(const uint4 *lds, f32x4 (&tmp)[RT][T
 // one tile and one token tile both sub-blocks' products are issued before the scale
 // multiplications (two independent chains); otherwise one sub-block at a time, whose
 // RT * TT chains already overlap (and keep the register count down).
-template <int TT, int RT>
-__device__ __forceinline__ void mma_pair(const f16x8 (&A)[TT][2][2], const f16x8 (&B)[RT][2], const float (&a)[RT][8],
+template <int NP, int TT, int RT>
+__device__ __forceinline__ void mma_pair(const f16x8 (&A)[TT][2][NP], const f16x8 (&B)[RT][2], const float (&a)[RT][8],
                                          int j0, bool add, f32x4 (&tmp)[RT][TT]) {
     constexpr int G = RT * TT == 1 ? 2 : 1;  // sub-blocks per group of products
 #pragma unroll
@@ -750,14 +773,15 @@ __device__ __forceinline__ void mma_pair(const f16x8 (&A)[TT][2][2], const f16x8
                 for (int t = 0; t < TT; t++)
                     D[i][v][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][u0 + v][0], B[i][u0 + v],
                                                                         (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if constexpr (NP == 2)
 #pragma unroll
-        for (int i = 0; i < RT; i++)
+            for (int i = 0; i < RT; i++)
 #pragma unroll
-            for (int v = 0; v < G; v++)
+                for (int v = 0; v < G; v++)
 #pragma unroll
-                for (int t = 0; t < TT; t++)
-                    D[i][v][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][u0 + v][1], B[i][u0 + v], D[i][v][t], 0,
-                                                                        0, 0);
+                    for (int t = 0; t < TT; t++)
+                        D[i][v][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][u0 + v][1], B[i][u0 + v], D[i][v][t],
+                                                                            0, 0, 0);
 #pragma unroll
         for (int i = 0; i < RT; i++)
 #pragma unroll
@@ -777,8 +801,8 @@ __device__ __forceinline__ void mma_pair(const f16x8 (&A)[TT][2][2], const f16x8
 // nibbles' sub-blocks) and the min coefficients -dmin m_j of sub-blocks kg, kg + 4.
 // Per 64-element group g, every (tile, sub-block, token tile) product is issued before
 // the scale multiplications that use them, so the matrix products overlap.
-template <int TT, int RT>
-__device__ __forceinline__ void q4k_chunk(const uint4 *lds, const Q4kChunk<RT> &W, float (&acc)[RT][TT][4]) {
+template <int NP, int TT, int RT, int TA>
+__device__ __forceinline__ void q4k_chunk(const uint4 *lds, const Q4kChunk<RT> &W, float (&acc)[RT][TA][4], int ta) {
     const uint32_t l = threadIdx.x & 63u, kg = l >> 4;
     float a[RT][8], cm[RT][2];
 #pragma unroll
@@ -804,15 +828,15 @@ __device__ __forceinline__ void q4k_chunk(const uint4 *lds, const Q4kChunk<RT> &
     f32x4 tmp[RT][TT];
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-        f16x8 A[TT][2][2];
+        f16x8 A[TT][2][NP];
 #pragma unroll
         for (int t = 0; t < TT; t++)
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
-                for (int p = 0; p < 2; p++)
+                for (int p = 0; p < NP; p++)
                     A[t][u][p] = __builtin_bit_cast(
-                        f16x8, lds[t * FR_U4 + ((2 * g + u) * 2 + p) * 64 + (l ^ (2 * (2 * g + u) + (l >> 5)))]);
+                        f16x8, lds[t * Fr<NP>::U4 + ((2 * g + u) * NP + p) * 64 + (l ^ (2 * (2 * g + u) + (l >> 5)))]);
         f16x8 B[RT][2];
 #pragma unroll
         for (int i = 0; i < RT; i++) {
@@ -820,15 +844,15 @@ __device__ __forceinline__ void q4k_chunk(const uint4 *lds, const Q4kChunk<RT> &
             B[i][0] = as_f16x8(v0 & LO4, u0 & LO4, v1 & LO4, u1 & LO4);
             B[i][1] = as_f16x8(v0 & HI4, u0 & HI4, v1 & HI4, u1 & HI4);
         }
-        mma_pair<TT, RT>(A, B, a, 2 * g, g > 0, tmp);
+        mma_pair<NP, TT, RT>(A, B, a, 2 * g, g > 0, tmp);
     }
-    chunk_close<TT, RT>(lds, tmp, cm, acc);
+    chunk_close<NP, TT, RT, TA>(lds, tmp, cm, acc, ta);
 }
 
 // One Q8_0 chunk: a_j = 2^24 d_j, bias coefficients -128 d_j of blocks kg, kg + 4.
 // Per pair of blocks, the products are issued before the scale multiplications.
-template <int TT, int RT, bool BIASED>
-__device__ __forceinline__ void q80_chunk(const uint4 *lds, const Q80Chunk<RT> &W, float (&acc)[RT][TT][4]) {
+template <int NP, int TT, int RT, bool BIASED, int TA>
+__device__ __forceinline__ void q80_chunk(const uint4 *lds, const Q80Chunk<RT> &W, float (&acc)[RT][TA][4], int ta) {
     const uint32_t l = threadIdx.x & 63u, kg = l >> 4;
     float a[RT][8], cm[RT][2];
 #pragma unroll
@@ -844,15 +868,15 @@ __device__ __forceinline__ void q80_chunk(const uint4 *lds, const Q80Chunk<RT> &
     f32x4 tmp[RT][TT];
 #pragma unroll
     for (int jp = 0; jp < 4; jp++) {
-        f16x8 A[TT][2][2];
+        f16x8 A[TT][2][NP];
 #pragma unroll
         for (int t = 0; t < TT; t++)
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
-                for (int p = 0; p < 2; p++)
+                for (int p = 0; p < NP; p++)
                     A[t][u][p] = __builtin_bit_cast(
-                        f16x8, lds[t * FR_U4 + ((2 * jp + u) * 2 + p) * 64 + (l ^ (2 * (2 * jp + u) + (l >> 5)))]);
+                        f16x8, lds[t * Fr<NP>::U4 + ((2 * jp + u) * NP + p) * 64 + (l ^ (2 * (2 * jp + u) + (l >> 5)))]);
         f16x8 B[RT][2];
 #pragma unroll
         for (int i = 0; i < RT; i++)
@@ -863,9 +887,9 @@ __device__ __forceinline__ void q80_chunk(const uint4 *lds, const Q80Chunk<RT> &
                 const uint32_t v0 = W.qv[i][2 * jp + u].x ^ bias, v1 = W.qv[i][2 * jp + u].y ^ bias;
                 B[i][u] = as_f16x8(v0 & LO8, (v0 >> 8) & LO8, v1 & LO8, (v1 >> 8) & LO8);
             }
-        mma_pair<TT, RT>(A, B, a, 2 * jp, jp > 0, tmp);
+        mma_pair<NP, TT, RT>(A, B, a, 2 * jp, jp > 0, tmp);
     }
-    chunk_close<TT, RT>(lds, tmp, cm, acc);
+    chunk_close<NP, TT, RT, TA>(lds, tmp, cm, acc, ta);
 }
 
 // The small-M product.  Wavefront w owns row tiles (4*bx + w)*RT .. +RT-1 (GLU: gate
@@ -881,14 +905,20 @@ constexpr uint32_t mm_spw() {
     return RT * 16 * (Q4 ? Q4K_PIECES : Q80_PIECES);
 }
 
-// The product of job J_ over TT token tiles; lrec holds two records of TT tiles,
-// lstage (raw blocks) 4 mm_spw<Q4, RT>() pieces.
+// The product of job J_ over TT token tiles; lrec holds two records of at most two tiles,
+// lstage (raw blocks) 4 mm_spw<Q4, RT>() pieces.  Three and four tiles run as two passes
+// over each chunk's weights, tiles 0-1 through the first record and the rest through the
+// second (a barrier each), so that the weights are read from memory once: Q8_0 tiles 4096 ->
+// 4099 at m = 61 (bf16) 30.8 -> 21.6 us against two launches of two tiles, Q4_K tiles 14336
+// -> 4096 at m = 64 (f32) 48.5 -> 38.9.
 template <bool Q4, int TT, int RT, bool GLU, bool NORM, bool TILED, int XM>
 __device__ __forceinline__ void mm_body(const void *x, const float *up, const MmJobs &jobs, uint32_t J_, uint32_t *cnt,
                                         uint32_t m, uint32_t k, uint64_t row_bytes, uint32_t ch, uint4 *lrec_base,
                                         lg_u32x4 *lstage) {
+    constexpr int T0 = TT > 2 ? 2 : TT, T1 = TT - T0, NP = XM == 1 ? 1 : 2;
+    static_assert(T1 == 0 || XM != 2, "three and four token tiles: plain activations");
     MM_JOB_FIELDS;
-    uint4 (*lrec)[TT * FR_U4] = reinterpret_cast<uint4 (*)[TT * FR_U4]>(lrec_base);
+    uint4 (*lrec)[T0 * Fr<NP>::U4] = reinterpret_cast<uint4 (*)[T0 * Fr<NP>::U4]>(lrec_base);
     // uniform over the wavefront: row-tile addresses are scalar
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t rt0 = (GLU ? bx * 2 + (wave & 1u) : bx * 4 + wave) * RT;
@@ -916,51 +946,68 @@ __device__ __forceinline__ void mm_body(const void *x, const float *up, const Mm
         for (int t = 0; t < TT; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[i][t][r] = 0.0f;
-    RecBuild<TT, XM> rb;
-    rb.load(x, up, m, k, c0);
+    RecBuild<T0, XM> rb;
+    RecBuild<T1 ? T1 : 1, XM> rb1;  // T1: tokens 32 ..
+    const void *x1 = static_cast<const uint8_t *>(x) + (uint64_t)32 * k * (XM == 1 ? 2 : 4);
+    const uint32_t m0 = T1 ? 32u : m, m1 = T1 ? m - 32 : 1u;
+    rb.load(x, up, m0, k, c0);
+    if constexpr (T1 > 0) rb1.load(x1, up, m1, k, c0);
     load_w(Wc[0], 0);
     load_w(Wc[1], 1);
-    // chunk 0 ahead of the loop, so the loop is entered in the state it repeats
-    rb.store(lrec[0], m);
-    __syncthreads();
-    rb.load(x, up, m, k, c0 + (1 < nch ? 1 : 0));
-    __builtin_amdgcn_sched_barrier(0);  // issue order: the activations, then the weights
-    load_w(Wc[2], 2);
-    __builtin_amdgcn_sched_barrier(0);
-    auto chunk = [&](const uint4 *rec, const Chunk &Wk) {
+    // chunk c's record stored, the activations of chunk c + 1 and the weights of chunk c + 2
+    // (into Wn) issued, chunk c (weights Wk) multiplied
+    auto step = [&](uint32_t c, Chunk &Wn, const Chunk &Wk) __attribute__((always_inline)) {
+        const uint32_t b = T1 ? 0u : c & 1u, cn = c0 + (c + 1 < nch ? c + 1 : nch - 1);
+        rb.store(lrec[b], m0);
+        __syncthreads();
+        rb.load(x, up, m0, k, cn);
+        __builtin_amdgcn_sched_barrier(0);  // issue order: the activations, then the weights
+        load_w(Wn, c + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        auto passes = [&](const auto &Ws, auto mul) __attribute__((always_inline)) {
+            mul(std::integral_constant<int, T0>{}, lrec[b], Ws, 0);
+            if constexpr (T1 > 0) {
+                rb1.store(lrec[1], m1);
+                __syncthreads();
+                rb1.load(x1, up, m1, k, cn);
+                __builtin_amdgcn_sched_barrier(0);
+                mul(std::integral_constant<int, T1>{}, lrec[1], Ws, T0);
+            }
+        };
+        auto mul4 = [&](auto tt, const uint4 *rec, const Q4kChunk<RT> &Ws, int ta) __attribute__((always_inline)) {
+            q4k_chunk<NP, decltype(tt)::value, RT, TT>(rec, Ws, acc, ta);
+        };
+        auto mul8 = [&](auto tt, const uint4 *rec, const Q80Chunk<RT> &Ws, int ta) __attribute__((always_inline)) {
+            q80_chunk<NP, decltype(tt)::value, RT, TILED, TT>(rec, Ws, acc, ta);
+        };
         if constexpr (RAW4) {
             Q4kChunk<RT> Ws;
             stage_q4k<RT>(Wk, Ws, lstage + wave * SPW);
-            q4k_chunk<TT, RT>(rec, Ws, acc);
+            passes(Ws, mul4);
         } else if constexpr (Q4) {
-            q4k_chunk<TT, RT>(rec, Wk, acc);
+            passes(Wk, mul4);
         } else if constexpr (RAW8) {
             Q80Chunk<RT> Ws;
             stage_q80<RT>(Wk, Ws, lstage + wave * SPW);
-            q80_chunk<TT, RT, false>(rec, Ws, acc);
+            passes(Ws, mul8);
         } else {
-            q80_chunk<TT, RT, TILED>(rec, Wk, acc);
+            passes(Wk, mul8);
         }
     };
-    chunk(lrec[0], Wc[0]);
-    // three chunks per iteration, so the ring's registers are named at compile time
-    // (chunk c in Wc[c % 3]: ci = 1 mod 3)
+    // chunk 0 ahead of the loop, so the loop is entered in the state it repeats; three
+    // chunks per iteration, so the ring's registers are named at compile time (chunk c in
+    // Wc[c % 3]: ci = 1 mod 3)
+    step(0, Wc[2], Wc[0]);
     for (uint32_t ci = 1; ci < nch; ci += 3) {
 #pragma unroll
         for (int h = 0; h < 3; h++) {
-            const uint32_t c = ci + h;
-            if (c >= nch) break;  // uniform
-            rb.store(lrec[c & 1u], m);
-            __syncthreads();
-            rb.load(x, up, m, k, c0 + (c + 1 < nch ? c + 1 : nch - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            load_w(Wc[h], c + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            chunk(lrec[c & 1u], Wc[(h + 1) % 3]);
+            if (ci + h >= nch) break;  // uniform
+            step(ci + h, Wc[h], Wc[(h + 1) % 3]);
         }
     }
-    static_assert(!GLU || 2 * RT * TT * 256 * 4 <= 2 * TT * FR_U4 * 16, "GLU exchange fits in the record LDS");
-    static_assert(RT != 2 || 8 * TT * 256 * 4 <= 2 * TT * FR_U4 * 16, "the head exchange fits in the record LDS");
+    constexpr int LREC = 2 * T0 * (int)Fr<NP>::U4 * 16;  // bytes
+    static_assert(!GLU || 2 * RT * TT * 256 * 4 <= LREC, "GLU exchange fits in the record LDS");
+    static_assert(RT != 2 || 8 * TT * 256 * 4 <= LREC || XM, "the head exchange fits in the record LDS");
     finish<TT, RT, GLU, NORM>(acc, out, res, part, cnt, rt0, m, n, reinterpret_cast<float *>(lrec_base), jobs, k,
                               jobs.j[J_].y, jobs.j[J_].yw, jobs.j[J_].ss, bx, jobs.j[J_].qkw);
 }
@@ -969,26 +1016,28 @@ template <bool Q4, int TT, int RT, bool GLU, bool NORM, bool TILED, int XM>
 __global__ __launch_bounds__(256) void k_mm_mf(const void *x, const float *up, MmJobs jobs, uint32_t *cnt, uint32_t m,
                                                uint32_t k, uint64_t row_bytes, uint32_t ch) {
     MM_JOB_INDEX;
-    __shared__ uint4 lrec[2 * TT * FR_U4];
+    __shared__ uint4 lrec[2 * (TT > 2 ? 2 : TT) * Fr<XM == 1 ? 1 : 2>::U4];
     __shared__ lg_u32x4 lstage[TILED ? 1 : 4 * mm_spw<Q4, RT>()];
-    if constexpr (TT == 2 && !GLU && XM == 0) {
-        if (jobs.j[J_].tlo) {  // uniform: this job takes token rows 16 .. m - 1 only (one tile)
+    if constexpr (TT >= 2 && !GLU && XM == 0) {
+        constexpr int SK = TT == 2 ? 1 : 2;  // tiles a job with tlo skips
+        if (jobs.j[J_].tlo) {  // uniform: this job takes token rows 16 SK .. m - 1 only
             // a launch of that one job, held as job 0 (static indices: no private copy)
+            constexpr uint32_t R0 = 16 * SK;
             MmJobs j1;
             j1.j[0] = jobs.j[J_];
-            j1.j[0].out += (uint64_t)16 * j1.j[0].n;
-            if (j1.j[0].res) j1.j[0].res += (uint64_t)16 * j1.j[0].n;
+            j1.j[0].out += (uint64_t)R0 * j1.j[0].n;
+            if (j1.j[0].res) j1.j[0].res += (uint64_t)R0 * j1.j[0].n;
             j1.count = 1;
             j1.tiled = jobs.tiled;
             j1.rs_cols = jobs.rs_cols;
             j1.rs_eps = jobs.rs_eps;
-            // the folded norm's rows, relative to the tile
-            j1.rs_ss = jobs.rs_ss + (uint64_t)(jobs.rs_tok0 < 16 ? 16 - jobs.rs_tok0 : 0) * jobs.rs_cols;
-            j1.rs_tok0 = jobs.rs_tok0 > 16 ? jobs.rs_tok0 - 16 : 0;
-            j1.rope = jobs.rope ? jobs.rope + 16 * 128 : nullptr;
+            // the folded norm's rows, relative to the first tile
+            j1.rs_ss = jobs.rs_ss + (uint64_t)(jobs.rs_tok0 < R0 ? R0 - jobs.rs_tok0 : 0) * jobs.rs_cols;
+            j1.rs_tok0 = jobs.rs_tok0 > R0 ? jobs.rs_tok0 - R0 : 0;
+            j1.rope = jobs.rope ? jobs.rope + R0 * 128 : nullptr;
             j1.qk_eps = jobs.qk_eps;
-            mm_body<Q4, 1, RT, GLU, NORM, TILED, XM>(static_cast<const float *>(x) + (uint64_t)16 * k, up, j1, 0u, cnt,
-                                                     m - 16, k, row_bytes, ch, lrec, lstage);
+            mm_body<Q4, TT - SK, RT, GLU, NORM, TILED, XM>(static_cast<const float *>(x) + (uint64_t)R0 * k, up, j1, 0u,
+                                                           cnt, m - R0, k, row_bytes, ch, lrec, lstage);
             return;
         }
     }
@@ -1080,6 +1129,7 @@ MmShape mm_shape(int dtype, uint32_t k, uint32_t n, uint32_t m, bool glu, bool q
     if (ort) rt = ort >= 4 ? 4 : ort >= 2 ? 2 : 1;
     if (dtype != LG_Q4_K && rt > 2) rt = 2;  // register budget of the Q8_0 chunk
     if (m > 16 && rt > 2) rt = 2;
+    if (m > 32) rt = 1;  // two passes over a chunk: the register budget
     if (qk) rt = 2;  // whole heads of 128 rows per column
     while (epi && rt < 2 && (n + per * rt - 1) / (per * rt) > 64) rt *= 2;
     const uint32_t cols = (n + per * rt - 1) / (per * rt);
@@ -1107,10 +1157,11 @@ void launch_rt(uint32_t rt, dim3 grid, const void *x, const float *up, const MmJ
             LG_MM(4);
             return;
         }
-    if (rt == 2) {
-        LG_MM(2);
-        return;
-    }
+    if constexpr (TT <= 2)
+        if (rt == 2) {
+            LG_MM(2);
+            return;
+        }
     LG_MM(1);
 #undef LG_MM
 }
@@ -1119,13 +1170,25 @@ void launch_rt(uint32_t rt, dim3 grid, const void *x, const float *up, const MmJ
 template <bool Q4, bool GLU, bool NORM, int XM>
 void launch_tt(uint32_t tt, bool tiled, uint32_t rt, dim3 grid, const void *x, const float *up, const MmJobs &jobs,
                uint32_t *cnt, uint32_t m, uint32_t k, uint64_t rb, uint32_t ch, hipStream_t s) {
-    if (tt == 2) {
-        if (tiled) launch_rt<Q4, 2, GLU, NORM, true, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s);
-        else launch_rt<Q4, 2, GLU, NORM, false, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s);
-    } else {
-        if (tiled) launch_rt<Q4, 1, GLU, NORM, true, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s);
-        else launch_rt<Q4, 1, GLU, NORM, false, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s);
+#define LG_TT(T)                                                                                                \
+    if (tiled) launch_rt<Q4, T, GLU, NORM, true, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s);              \
+    else launch_rt<Q4, T, GLU, NORM, false, XM>(rt, grid, x, up, jobs, cnt, m, k, rb, ch, s)
+    if constexpr (XM != 2) {
+        if (tt == 4) {
+            LG_TT(4);
+            return;
+        }
+        if (tt == 3) {
+            LG_TT(3);
+            return;
+        }
     }
+    if (tt == 2) {
+        LG_TT(2);
+    } else {
+        LG_TT(1);
+    }
+#undef LG_TT
 }
 
 template <bool Q4>
@@ -1157,7 +1220,7 @@ uint64_t align256(uint64_t b) { return (b + 255) & ~(uint64_t)255; }
 constexpr uint64_t CNT_BYTES = PROJ_WS_COUNTERS;
 constexpr uint32_t CNT_MAX = CNT_BYTES / 4;
 
-// The shape of the launch over the token tiles 16 t0 .. (pairs of tiles; ml rows).
+// The shape of a launch over ml rows.
 MmShape launch_shape(int w_dtype, uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t ml, bool glu, bool qk,
                      bool epi) {
     uint64_t ntot = 0;
@@ -1177,18 +1240,27 @@ uint64_t mm_part_floats(uint32_t n, uint32_t ml, uint32_t rt, uint32_t slices, b
 
 namespace lg {
 
-// The workspace of one call: counters, partial sums of the largest tile pair, records.
-static uint64_t multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t m, int w_dtype, bool glu,
-                               bool qk, bool epi) {
-    if (w_dtype == LG_Q4_K_T16) w_dtype = LG_Q4_K;
-    if (w_dtype == LG_Q8_0_T16) w_dtype = LG_Q8_0;
-    if ((w_dtype != LG_Q4_K && w_dtype != LG_Q8_0) || k % QK_K || m == 0) return 0;
-    const uint32_t ml = m < 32 ? m : 32;
+// Rows of one launch: up to four token tiles, two for the fused SiLU input.
+static uint32_t launch_rows(bool up) { return up ? 32 : 64; }
+
+// The workspace of one call: counters and the partial sums of its largest launch.
+static uint64_t launch_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t ml, int w_dtype, bool glu,
+                                bool qk, bool epi) {
     const MmShape sh = launch_shape(w_dtype, k, n, jobs, ml, glu, qk, epi);
     uint64_t b = CNT_BYTES;
     if (sh.slices > 1)
         for (uint32_t j = 0; j < jobs; j++) b += align256(mm_part_floats(n[j], ml, sh.rt, sh.slices, glu) * 4);
     return b;
+}
+static uint64_t multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t m, int w_dtype, bool glu,
+                               bool qk, bool epi) {
+    if (w_dtype == LG_Q4_K_T16) w_dtype = LG_Q4_K;
+    if (w_dtype == LG_Q8_0_T16) w_dtype = LG_Q8_0;
+    if ((w_dtype != LG_Q4_K && w_dtype != LG_Q8_0) || k % QK_K || m == 0) return 0;
+    const uint64_t b = launch_ws_bytes(k, n, jobs, m < 64 ? m : 64, w_dtype, glu, qk, epi);
+    if (m <= 32) return b;
+    const uint64_t p = launch_ws_bytes(k, n, jobs, 32, w_dtype, glu, qk, epi);  // with the fused SiLU input
+    return b > p ? b : p;
 }
 
 uint64_t proj_batch_multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t m, int w_dtype) {
@@ -1220,7 +1292,7 @@ uint32_t proj_batch_norm_cols(int w_dtype, uint32_t k, uint32_t n, uint32_t m) {
     return (n + 64 * sh.rt - 1) / (64 * sh.rt);
 }
 
-uint32_t proj_batch_rs_cols_max(uint32_t m) { return MM_SS_LOADS * (m > 16 ? 8u : 16u); }
+uint32_t proj_batch_rs_cols_max(uint32_t m) { return m > 16 ? 64u : 128u; }
 
 bool proj_batch_mfma_ok(int w_dtype, uint32_t k, const void *w) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(w);
@@ -1327,8 +1399,9 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
     const uint32_t tiles = (m + 15) / 16;
     const uint64_t xsz = x_dtype == LG_F32 ? 4 : 2;
     const int xm = x_dtype == LG_BF16 ? 1 : (up ? 2 : 0);
-    for (uint32_t t0 = 0; t0 < tiles; t0 += 2) {  // pairs of 16-token tiles
-        const uint32_t ml = m - 16 * t0 < 32 ? m - 16 * t0 : 32, tt = (ml + 15) / 16;
+    const uint32_t lrows = launch_rows(up != nullptr);
+    for (uint32_t t0 = 0; t0 < tiles; t0 += lrows / 16) {
+        const uint32_t ml = m - 16 * t0 < lrows ? m - 16 * t0 : lrows, tt = (ml + 15) / 16;
         const MmShape sh = launch_shape(w_dtype, k, nv, njobs, ml, glu, qkn, epi);
         uint32_t *cnt = static_cast<uint32_t *>(ws);
         uint8_t *pb = static_cast<uint8_t *>(ws) + CNT_BYTES;
@@ -1336,8 +1409,9 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
         uint32_t groups = 0;
         for (uint32_t j = 0; j < njobs; j++) {
             const uint64_t off = (uint64_t)16 * t0 * jb[j].n;
-            // a job whose rows below 16 t0 + 16 are not needed skips the pair's first tile
-            const uint32_t tlo = tt == 2 && !glu && xm == 0 && !jb[j].ss && jb[j].row0 >= 16 * t0 + 16 ? 1u : 0u;
+            // a job whose rows below 16 t0 + 16 (three and four tiles: 16 t0 + 32) are not needed
+            // skips those tiles
+            const uint32_t tlo = tt >= 2 && !glu && xm == 0 && !jb[j].ss && jb[j].row0 >= 16 * (t0 + (tt == 2 ? 1 : 2)) ? 1u : 0u;
             jobs.j[j] = {static_cast<const uint8_t *>(jb[j].w), jb[j].c + off, jb[j].res ? jb[j].res + off : nullptr,
                          reinterpret_cast<float *>(pb), jb[j].y, jb[j].yw, jb[j].ss, jb[j].n, groups, jb[j].qkw, tlo};
             if (sh.slices > 1) pb += align256(mm_part_floats(jb[j].n, ml, sh.rt, sh.slices, glu) * 4);
@@ -1353,7 +1427,7 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
             jobs.rope = qk->table + (uint64_t)16 * t0 * 128;
             jobs.qk_eps = qk->eps;
         }
-        // the folded norm's scaled rows in this pair of tiles (rows 16 t0 .. 16 t0 + ml - 1)
+        // the folded norm's scaled rows in this launch (rows 16 t0 .. 16 t0 + ml - 1)
         const bool pnorm = norm && 16 * t0 + ml > rs->tok0;
         if (pnorm) {
             jobs.rs_tok0 = rs->tok0 > 16 * t0 ? rs->tok0 - 16 * t0 : 0u;
