@@ -29,8 +29,8 @@
 //
 // Q8_0 with k <= 4096: integer dot products against activation digits (k_q80_m1_dig,
 // described there).  Q8_0 with k > 4096, the fused path over Q8_0 and k no multiple of 256:
-// proj_q80_rows, up to its longest row.  Plain Q8_0 beyond that: vector ALU (k_q80_m1).  A
-// "team" of TW waves covers one row in passes of 4096 TW elements: lane p of
+// proj_q80_rows, up to its longest row.  Plain Q8_0 beyond that and where q80_team says so:
+// vector ALU (k_q80_m1).  A "team" of TW waves covers one row in passes of 4096 TW elements: lane p of
 // the team owns the 64-element group p of the row (two 34-byte blocks, 68 bytes,
 // dword aligned) and keeps the 64 activations of that group in registers; the
 // team's partial sums meet in a DPP/swizzle wavefront reduction (plus LDS across
@@ -1864,7 +1864,18 @@ int launch_q80(const float *x, const uint8_t *w, float *y, uint32_t k, uint32_t 
                            (uint64_t)k / QK8_0 * Q80_BYTES);
         return after_launch("proj_q8_0_m1", s);
     }
-    return launch_q80_t<4, 2>(x, w, y, k, n, s);  // past proj_q80_rows' longest row
+    return P <= 128 ? launch_q80_t<2, 4>(x, w, y, k, n, s) : launch_q80_t<4, 2>(x, w, y, k, n, s);
+}
+
+// Plain Q8_0, k a multiple of 256 above 4096: where a team per row beats proj_q80_rows
+// (activations in registers, each read once per team and not per row).  us, here against there:
+// 8192 -> 2048 5.9 / 6.3, -> 4096 10.1 / 11.7, -> 6144 14.3 / 17.2, -> 9000 46 / 25.8; 5120 ->
+// 3072 6.65 / 6.1, -> 6144 11.8 / 12.2; 16384 -> 1536 7.8 / 8.6, -> 2048 11.0 / 12.4, -> 3072
+// 20.1 / 16.3; 28672 -> 512 6.9 / 5.8, -> 1024 9.7 / 10.2; 12288 -> 2048 8.7 / 8.2
+bool q80_team(uint32_t k, uint32_t n) {
+    const uint64_t cus = (uint64_t)device_cus();
+    if (k <= 8192) return n >= (k >= 6144 ? 8 : 16) * cus && n <= 24 * cus;
+    return k > 12288 && n >= 4 * cus && n <= 8 * cus;
 }
 
 // Shared front end of every quantized M=1 entry point.
@@ -1913,7 +1924,7 @@ int proj_quant(const float *x, const float *up, const void *w, float *c, uint32_
     }
     if (dtype == LG_Q8_0) {
         const bool q80 = vec_ok && !fuse && aligned16(wb);
-        if (q80 && k <= 4096) return launch_q80(x, wb, c, k, n, s);
+        if (q80 && (k <= 4096 || q80_team(k, n))) return launch_q80(x, wb, c, k, n, s);
         if (proj_q80_rows_ok(k, n, x, up, wb)) return proj_q80_rows(x, up, wb, c, k, n, s);
         if (q80) return launch_q80(x, wb, c, k, n, s);
     }

@@ -99,6 +99,80 @@ __global__ __launch_bounds__(QR_WAVES * 64) void k_q80_rows(const float *__restr
     }
 }
 
+// Few rows: latency and idle CUs bound them, not bandwidth (16384 -> 275, 4.8 MB, is 16 steps of
+// one wavefront a row on 35 workgroups above).  The eight wavefronts of a workgroup share R
+// rows, thread t the half blocks t, t + 512, ..., its activations straight from memory (so few
+// readers pay for no staging); four rows a workgroup lost to two (16384 -> 1024 6.4 against 6.3
+// us, -> 512 6.0 against 4.3).
+template <int R, bool FUSE>
+__global__ __launch_bounds__(QR_WAVES * 64) void k_q80_split(const float *__restrict__ x, const float *__restrict__ up,
+                                                             const uint8_t *__restrict__ w, float *__restrict__ y,
+                                                             uint32_t k, uint32_t n) {
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t units = k / 16, row = blockIdx.x * R;
+    const uint64_t row_bytes = (uint64_t)k / QK8_0 * Q80_BYTES;
+    float acc[R][2];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r][0] = acc[r][1] = 0.0f;
+    for (uint32_t u0 = threadIdx.x; u0 < units; u0 += 2 * QR_WAVES * 64) {
+        u32x4a2 q[2][R];
+        uint32_t d[2][R];
+        float4 xv[2][4], uv[2][4];
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const uint32_t u = u0 + QR_WAVES * 64 * b < units ? u0 + QR_WAVES * 64 * b : u0;  // past the row: dropped
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint32_t rr = row + r < n ? row + r : n - 1;  // past n: not stored
+                const uint8_t *blk = w + rr * row_bytes + (uint64_t)(u >> 1) * Q80_BYTES;
+                d[b][r] = *reinterpret_cast<const uint16_t *>(blk);
+                q[b][r] = *reinterpret_cast<const u32x4a2 *>(blk + 2 + 16 * (u & 1u));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                xv[b][i] = reinterpret_cast<const float4 *>(x)[4 * u + i];
+                if constexpr (FUSE) uv[b][i] = reinterpret_cast<const float4 *>(up)[4 * u + i];
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if (u0 + QR_WAVES * 64 * b >= units) break;
+            float xe[16];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float4 v = xv[b][i];
+                if constexpr (FUSE) {
+                    const float4 u = uv[b][i];
+                    v = make_float4(silu_mul(v.x, u.x), silu_mul(v.y, u.y), silu_mul(v.z, u.z), silu_mul(v.w, u.w));
+                }
+                xe[4 * i] = v.x, xe[4 * i + 1] = v.y, xe[4 * i + 2] = v.z, xe[4 * i + 3] = v.w;
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float df = ref_half(d[b][r]);
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const float wv = __fmul_rn((float)(int8_t)(q[b][r][i >> 2] >> (8 * (i & 3))), df);
+                    acc[r][i & 1] = __builtin_fmaf(xe[i], wv, acc[r][i & 1]);
+                }
+            }
+        }
+    }
+    __shared__ float part[QR_WAVES][R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float s = wave_sum(acc[r][0] + acc[r][1]);
+        if (lane == 0) part[wave][r] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < R && row + threadIdx.x < n) {
+        float s = part[0][threadIdx.x];
+#pragma unroll
+        for (int v = 1; v < QR_WAVES; v++) s += part[v][threadIdx.x];
+        y[row + threadIdx.x] = s;
+    }
+}
+
 std::mutex g_mu;
 bool g_attr[64][2][2] = {};
 
@@ -132,9 +206,25 @@ bool proj_q80_rows_ok(uint32_t k, uint32_t n, const float *x, const float *up, c
 
 int proj_q80_rows(const float *x, const float *up, const void *w, float *y, uint32_t k, uint32_t n, hipStream_t s) {
     const uint8_t *wb = static_cast<const uint8_t *>(w);
+    // fewer rows than keep the chip busy at one wavefront each: a workgroup per row (a CU's
+    // worth of rows or less) or two.  Plain, 16384 -> 256 10.1 -> 3.9 us, -> 3072 18.3 -> 16.3,
+    // 5120 -> 3072 6.9 -> 6.1, -> 16000 21.7 against 24.7 here; fused, 14336 -> 1024 11.3 -> 10.4,
+    // -> 2048 11.5 against 20.8: each row repeats the SiLU
+    const uint32_t cus = (uint32_t)device_cus();
+    if (n < (up ? 4u * cus + 1 : 16u * cus)) {
+        const dim3 b(QR_WAVES * 64);
+        if (n <= cus) {
+            if (up) hipLaunchKernelGGL((k_q80_split<1, true>), dim3(n), b, 0, s, x, up, wb, y, k, n);
+            else hipLaunchKernelGGL((k_q80_split<1, false>), dim3(n), b, 0, s, x, up, wb, y, k, n);
+        } else {
+            if (up) hipLaunchKernelGGL((k_q80_split<2, true>), dim3((n + 1) / 2), b, 0, s, x, up, wb, y, k, n);
+            else hipLaunchKernelGGL((k_q80_split<2, false>), dim3((n + 1) / 2), b, 0, s, x, up, wb, y, k, n);
+        }
+        return after_launch("proj_q8_0_split", s);
+    }
     // two rows a wavefront share the reads of x once every CU has its eight wavefronts
-    if (n >= 16u * (uint32_t)device_cus()) return up ? launch<2, true>(x, up, wb, y, k, n, s) : launch<2, false>(x, up, wb, y, k, n, s);
-    return up ? launch<1, true>(x, up, wb, y, k, n, s) : launch<1, false>(x, up, wb, y, k, n, s);
+    if (!up) return launch<2, false>(x, up, wb, y, k, n, s);
+    return n >= 16u * cus ? launch<2, true>(x, up, wb, y, k, n, s) : launch<1, true>(x, up, wb, y, k, n, s);
 }
 
 }  // namespace lg

@@ -59,3 +59,26 @@ def test_q80_rows_nonfinite(ctx, fuse):
         assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
         ok = np.isfinite(a)
         assert np.allclose(a[ok], b[ok], rtol=1e-5, atol=1e-5) and np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+
+
+# rows shared by a workgroup's wavefronts, odd counts among them, a team of wavefronts per row,
+# and a wavefront per row or two, on both sides of each line between them (256 CUs); the longest
+# staged row
+@pytest.mark.parametrize("k,n,fuse", [
+    (4352, 256, 0), (4352, 257, 0), (8224, 1025, 0), (992, 4095, 0), (992, 4096, 0), (6144, 2047, 0), (6144, 2048, 0),
+    (5120, 4095, 0), (5120, 4096, 0), (5120, 6144, 0), (5120, 6145, 0), (12288, 1024, 0), (16384, 1023, 0),
+    (16384, 1024, 0), (16384, 2048, 0), (16384, 2049, 0), (32768, 1, 0), (33024, 5, 0), (4352, 256, 1), (4352, 257, 1),
+    (4128, 1024, 1), (4128, 1025, 1), (32224, 1026, 1)])
+def test_q80_few_rows(ctx, k, n, fuse):
+    print(f"q8_0 few rows k={k} n={n} fuse={fuse}", flush=True)
+    raw = synth.q8_0_weight(0x5EED0A20 + k, k, n)
+    x = synth.normal(0x5EED0A21 + n, k)
+    up = synth.normal(0x5EED0A22 + n, k) if fuse else None
+    y = call(ctx, raw, x, up, k, n)
+    h = x.astype(np.float64) if up is None else x.astype(np.float64) / (1.0 + np.exp(-x.astype(np.float64))) * up
+    y64, a = orc.proj_quant_f64(h.astype(np.float32), raw, lh.Q8_0, k, n)
+    # of the sum of magnitudes: the product's two roundings and the input's (the SiLU's four with
+    # it), a lane's chain of at most 64 additions for each 4096 elements of its row (a lane takes
+    # 64 of them), and the sums over lanes and wavefronts
+    assert np.all(np.abs(y - y64) <= (8 + 64 * (1 + k // 4096) + 16) * 2.0 ** -24 * a)
+    assert np.max(np.abs(y - y64) / a) <= 1e-6
