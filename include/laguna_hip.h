@@ -193,8 +193,8 @@ int lg_dispatch_proj_quant_batch_static(const void *x, int x_dtype, const void *
  * counterpart in the reference.  It is 64 KiB of arrival counters plus, when the
  * product splits k over slices, the split-k partial sums: slices * n' * 16 * tiles * 4
  * bytes, n' = n rounded up to whole workgroup columns (64 or 128 rows) and tiles =
- * ceil(m / 16) (slices chosen for about two workgroups per CU; the larger of this and
- * m = 32 for m > 32).
+ * ceil(m / 16) (slices chosen for about two workgroups per CU; the largest over the launches
+ * of at most 32 or 64 rows that m is taken in).
  * lg_dispatch_proj_quant_batch_static accepts a shape when this is at most
  * 16 MiB + 64 KiB. */
 uint64_t lg_proj_quant_batch_ws_bytes(uint32_t k, uint32_t n, uint32_t m, int w_dtype);

@@ -1100,10 +1100,8 @@ __global__ __launch_bounds__(256) void k_generic_batch(const void *__restrict__ 
     }
 }
 
-// Launch shape: RT 16-row tiles per wavefront, `ch` chunks of 256 elements per k
-// slice, `slices` = ceil(nb / ch) workgroup rows.  Automatic choice: RT = 2 (RT = 1
-// when that gives fewer than 256 workgroup columns... see mm_shape), and slices so
-// that columns x slices is about MM_TARGET_PER_CU workgroups per compute unit.
+// Launch shape: RT 16-row tiles per wavefront, `ch` chunks of 256 elements per k slice,
+// `slices` = ceil(nb / ch) workgroup rows (mm_shape).
 struct MmShape {
     uint32_t ch, slices, rt;
 };
@@ -1111,35 +1109,71 @@ struct MmShape {
 std::atomic<uint32_t> g_mm_ch{0}, g_mm_rt{0};  // launch-shape overrides (0 = automatic)
 constexpr uint32_t MM_TARGET_PER_CU = 2;
 
-// n: rows per workgroup column's job span (the jobs' total rows; a gate/up pair's n);
-// rows_per_wave_tile: 16.  glu: both products in every column (32 RT rows each).
-// epi: the job writes a folded norm's per-column sums of squares, whose consumers read
-// at most proj_batch_rs_cols_max partial sums per token: at most 64 columns.
-MmShape mm_shape(int dtype, uint32_t k, uint32_t n, uint32_t m, bool glu, bool qk, bool epi = false) {
-    const uint32_t nb = k / QK_K;
-    const uint32_t cus = (uint32_t)device_cus(), target = MM_TARGET_PER_CU * cus;
+// n: rows per workgroup column's job span (the jobs' total rows; a gate/up pair's n).
+// glu: both products in every column (32 RT rows each).  epi: the job writes a folded norm's
+// per-column sums of squares, whose consumers read at most proj_batch_rs_cols_max partial
+// sums per token: at most 64 columns.
+//
+// The slices follow from (dtype, k, n, m) alone: products over tiles or of bf16 activations
+// add their slices as those over raw blocks and of f32 do.  Figures: us per product, k = 4096
+// unless stated, the other choice -> the one taken.
+MmShape mm_shape(int dtype, bool tiled, uint32_t k, uint32_t n, uint32_t m, bool glu, bool qk, bool epi) {
+    const uint32_t nb = k / QK_K, cus = (uint32_t)device_cus();
     const uint32_t per = glu ? 32u : 64u;  // rows per column and row tile per wavefront
-    uint32_t rt = 2;
-    if ((n + per * 2 - 1) / (per * 2) < cus / 4) rt = 1;
-    // a gate/up pair with at least one RT = 1 column per CU: no k split, so no partial
-    // sums and no finishing workgroup (the draft's 14336-row pair: 448 columns of whole
-    // k against 224 x 2 slices, 610.2 -> 604.9 us per block forward)
-    if (glu && m <= 16 && (n + per - 1) / per >= cus) rt = 1;
+    const uint32_t c1 = (n + per - 1) / per, c2 = (n + 2 * per - 1) / (2 * per);  // columns at RT = 1, 2
+    const bool q4 = dtype == LG_Q4_K, few = c2 < cus / 4;
+    // a gate/up pair of short rows and about a column per CU takes all of k in each: no partial
+    // sums, no finishing workgroup (2 x 7168 x 2048 tiles, m = 16: Q4_K 11.7 -> 10.4, Q8_0 15.9 ->
+    // 12.5; m = 64 Q4_K 26.7 against 28.1).  Long rows want the second workgroup per CU more
+    // (2 x 8192, m = 16 Q4_K: two slices 17.3, whole 18.4).
+    const bool whole = glu && nb <= 8 && c1 >= cus * 7 / 8 && c1 <= cus && (!q4 || m <= 32);
+    uint32_t rt, rs;  // row tiles; those the slices are counted over
+    if (m > 32 || whole) rt = 1;  // above 32 rows two passes over a chunk: the register budget
+    else if (few || epi) rt = 1;
+    // RT = 1: no k split from a column per CU on (the draft's 14336-row pair, m = 16: 448
+    // columns of whole k against 224 x 2 slices, 610.2 -> 604.9 per block forward); Q8_0 always
+    // (2 x 7168 x 2048 tiles, m = 32 25.1 -> 18.4)
+    else if (glu) rt = !q4 || (m <= 16 && c1 >= cus) ? 1 : 2;
+    // up to 16 rows more workgroups hide more latency (n = 14336, m = 16: Q8_0 raw 29.5 -> 23.0,
+    // tiles 23.9 -> 21.5, Q4_K tiles 17.6 -> 16.7), Q4_K up to a column per CU (20000: 23.9 ->
+    // 21.5 with RT = 2; 151936: 141 -> 121)
+    else if (m <= 16) rt = q4 && c1 > cus ? 2 : 1;
+    // 17 to 32 rows: Q8_0 tiles RT = 1 (n = 14336, m = 32 39.8 -> 29.5), raw Q8_0 RT = 2 (40.9 ->
+    // 35.9); Q4_K tiles RT = 2 (25.8 -> 24.8), raw RT = 1 (33.0 -> 26.9) but for a head of at
+    // least 7/8 column per CU (30000: 45.4 -> 43.2)
+    else rt = tiled == q4 || (q4 && c2 >= cus * 7 / 8) ? 2 : 1;
+    rs = !glu && !epi && m > 16 && m <= 32 ? (q4 && !few ? 2 : 1) : rt;
     const uint32_t ort = g_mm_rt.load(std::memory_order_relaxed);
     if (ort) rt = ort >= 4 ? 4 : ort >= 2 ? 2 : 1;
-    if (dtype != LG_Q4_K && rt > 2) rt = 2;  // register budget of the Q8_0 chunk
+    if (!q4 && rt > 2) rt = 2;  // register budget of the Q8_0 chunk
     if (m > 16 && rt > 2) rt = 2;
-    if (m > 32) rt = 1;  // two passes over a chunk: the register budget
+    if (m > 32) rt = 1;
     if (qk) rt = 2;  // whole heads of 128 rows per column
     while (epi && rt < 2 && (n + per * rt - 1) / (per * rt) > 64) rt *= 2;
-    const uint32_t cols = (n + per * rt - 1) / (per * rt);
-    // two token tiles of two row tiles take every register of a SIMD (one workgroup per
-    // CU): about 9/8 workgroups per CU instead (the 32-row K/V/Q launch of the draft
-    // block: 610 against 624 us per block forward with 2 per CU, 614 with 3/4 per CU)
-    const uint32_t tgt = m > 16 && rt == 2 ? cus * 9 / 8 : target;
-    uint32_t slices = (tgt + cols / 2) / cols;
+    if (ort || qk || epi) rs = rt;
+    const uint32_t cols = (n + per * rs - 1) / (per * rs);
+    // slices: about MM_TARGET_PER_CU workgroups per CU; about 9/8 for the draft's 32-row K/V/Q
+    // launch, whose workgroups take every register of a CU (its block 610 against 624 with two
+    // per CU, 614 with 3/4), and for a 17 to 32-row Q4_K head of at least 7/8 column per CU
+    const bool nine8 = m > 16 && rs == 2 && (qk || epi || (!glu && c2 >= cus * 7 / 8));
+    const uint32_t tgt = nine8 ? cus * 9 / 8 : MM_TARGET_PER_CU * cus;
+    uint32_t slices = whole ? 1 : (tgt + cols / 2) / cols;
+    if (!q4 && m > 48) {
+        // the record of more than 48 f32 rows leaves a CU's LDS to one workgroup: the split whose
+        // rounds over the CUs take the fewest chunks, two more for each round's start and finish,
+        // and never more slices (partial sums) than two workgroups per CU make (m = 64 tiles: n = 14336 60.7 -> 54.4 with one slice, n = 4096 24.2 -> 20.9 with four)
+        uint32_t best = ~0u;
+        for (uint32_t t = 1, most = slices; t <= nb && t <= (most ? most : 1); t++) {
+            const uint32_t cost = (cols * t + cus - 1) / cus * ((nb + t - 1) / t + 2);
+            if (cost < best) best = cost, slices = t;
+        }
+    }
     slices = slices < 1 ? 1 : (slices > nb ? nb : slices);
     uint32_t ch = nb ? (nb + slices - 1) / slices : 1;
+    // a slice of one chunk pays its finish for a single step: two where eight slices or more are
+    // left (n = 1024, m = 16 Q4_K tiles 8.0 -> 7.1, n = 2048 8.5 -> 7.1; of four, k = n = 2048,
+    // 6.1 against 6.4)
+    if (ch == 1 && nb >= 16) ch = 2;
     const uint32_t och = g_mm_ch.load(std::memory_order_relaxed);
     if (och) ch = och < nb ? och : (nb ? nb : 1);
     ch = ch ? ch : 1;
@@ -1221,11 +1255,11 @@ constexpr uint64_t CNT_BYTES = PROJ_WS_COUNTERS;
 constexpr uint32_t CNT_MAX = CNT_BYTES / 4;
 
 // The shape of a launch over ml rows.
-MmShape launch_shape(int w_dtype, uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t ml, bool glu, bool qk,
-                     bool epi) {
+MmShape launch_shape(int w_dtype, bool tiled, uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t ml,
+                     bool glu, bool qk, bool epi) {
     uint64_t ntot = 0;
     for (uint32_t j = 0; j < jobs; j++) ntot += n[j];
-    return mm_shape(w_dtype, k, glu ? n[0] : (uint32_t)ntot, ml, glu, qk, epi);
+    return mm_shape(w_dtype, tiled, k, glu ? n[0] : (uint32_t)ntot, ml, glu, qk, epi);
 }
 
 // Floats of one job's split-k partials (finish): per workgroup column and slice, four
@@ -1243,24 +1277,37 @@ namespace lg {
 // Rows of one launch: up to four token tiles, two for the fused SiLU input.
 static uint32_t launch_rows(bool up) { return up ? 32 : 64; }
 
-// The workspace of one call: counters and the partial sums of its largest launch.
+// The workspace of one call: counters and the partial sums of its largest launch, over raw
+// blocks or tiles.
 static uint64_t launch_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t ml, int w_dtype, bool glu,
                                 bool qk, bool epi) {
-    const MmShape sh = launch_shape(w_dtype, k, n, jobs, ml, glu, qk, epi);
-    uint64_t b = CNT_BYTES;
-    if (sh.slices > 1)
-        for (uint32_t j = 0; j < jobs; j++) b += align256(mm_part_floats(n[j], ml, sh.rt, sh.slices, glu) * 4);
-    return b;
+    uint64_t most = 0;
+    // the layout matters only to plain products of 17 to 32 rows (mm_shape)
+    for (int v = 0; v < (ml > 16 && ml <= 32 && !glu && !qk ? 2 : 1); v++) {
+        const MmShape sh = launch_shape(w_dtype, v != 0, k, n, jobs, ml, glu, qk, epi);
+        uint64_t b = CNT_BYTES;
+        if (sh.slices > 1)
+            for (uint32_t j = 0; j < jobs; j++) b += align256(mm_part_floats(n[j], ml, sh.rt, sh.slices, glu) * 4);
+        most = b > most ? b : most;
+    }
+    return most;
 }
 static uint64_t multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t m, int w_dtype, bool glu,
                                bool qk, bool epi) {
     if (w_dtype == LG_Q4_K_T16) w_dtype = LG_Q4_K;
     if (w_dtype == LG_Q8_0_T16) w_dtype = LG_Q8_0;
     if ((w_dtype != LG_Q4_K && w_dtype != LG_Q8_0) || k % QK_K || m == 0) return 0;
-    const uint64_t b = launch_ws_bytes(k, n, jobs, m < 64 ? m : 64, w_dtype, glu, qk, epi);
-    if (m <= 32) return b;
-    const uint64_t p = launch_ws_bytes(k, n, jobs, 32, w_dtype, glu, qk, epi);  // with the fused SiLU input
-    return b > p ? b : p;
+    // full launches of launch_rows rows, with the fused SiLU input or without, and their rest
+    uint64_t most = 0;
+    uint32_t done = 0;  // m <= 32 is one launch either way: computed once, this is on each call's path
+    for (uint32_t rows : {launch_rows(true), launch_rows(false)})
+        for (uint32_t ml : {m < rows ? m : rows, m % rows})
+            if (ml && ml != done) {
+                const uint64_t b = launch_ws_bytes(k, n, jobs, ml, w_dtype, glu, qk, epi);
+                most = b > most ? b : most;
+                done = ml;
+            }
+    return most;
 }
 
 uint64_t proj_batch_multi_ws_bytes(uint32_t k, const uint32_t *n, uint32_t jobs, uint32_t m, int w_dtype) {
@@ -1286,9 +1333,10 @@ uint64_t proj_batch_ws_bytes(uint32_t k, uint32_t n, uint32_t m, int x_dtype, in
 }
 
 uint32_t proj_batch_norm_cols(int w_dtype, uint32_t k, uint32_t n, uint32_t m) {
+    const bool tiled = w_dtype == LG_Q4_K_T16 || w_dtype == LG_Q8_0_T16;
     if (w_dtype == LG_Q4_K_T16) w_dtype = LG_Q4_K;
     if (w_dtype == LG_Q8_0_T16) w_dtype = LG_Q8_0;
-    const MmShape sh = mm_shape(w_dtype, k, n, m < 32 ? m : 32, false, false, true);
+    const MmShape sh = mm_shape(w_dtype, tiled, k, n, m < 32 ? m : 32, false, false, true);
     return (n + 64 * sh.rt - 1) / (64 * sh.rt);
 }
 
@@ -1402,7 +1450,7 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
     const uint32_t lrows = launch_rows(up != nullptr);
     for (uint32_t t0 = 0; t0 < tiles; t0 += lrows / 16) {
         const uint32_t ml = m - 16 * t0 < lrows ? m - 16 * t0 : lrows, tt = (ml + 15) / 16;
-        const MmShape sh = launch_shape(w_dtype, k, nv, njobs, ml, glu, qkn, epi);
+        const MmShape sh = launch_shape(w_dtype, tiled, k, nv, njobs, ml, glu, qkn, epi);
         uint32_t *cnt = static_cast<uint32_t *>(ws);
         uint8_t *pb = static_cast<uint8_t *>(ws) + CNT_BYTES;
         MmJobs jobs{};
