@@ -1626,9 +1626,10 @@ uint32_t attn_split_chunks(uint32_t S, uint32_t groups) {
     return nch ? nch : 1;
 }
 
-// The attention workspace: arrival counters first (k_attn_split's, one per query group,
-// zero between calls), then the partials of whichever kernel runs.
-uint32_t attn_cnt_floats(uint32_t n_kv) { return (4 * n_kv + 63) / 64 * 64; }
+// k_attn_split's arrival counters (one per query group, at most 4 per kv head; zero between
+// calls) have a region of a fixed size at a fixed place of whatever memory holds them, so
+// that no call of other head counts writes its partials there.
+constexpr uint32_t ATTN_COUNTERS = (uint32_t)(PROJ_WS_COUNTERS / 4);
 
 // k_attn_rows: head sizes it is built for; more than AQ queries per kv head of AHD (up to
 // there k_attn_split and the few-query kernels), any number of the other sizes.
@@ -1669,7 +1670,7 @@ size_t attn_partial_floats(uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_k
     const uint64_t cap = (S + RPT - 1) / RPT, wg = groups * (cap < 64 ? cap : 64);
     const size_t many = hd == 64 || hd == AHD || hd == 256 ? (wg < cus ? wg : cus) * RQB * (hd + 2) : 0;
     const size_t few = decode > split ? decode : split;
-    return attn_cnt_floats(n_kv) + (many > few ? many : few);
+    return many > few ? many : few;
 }
 
 template <int HD>
@@ -1692,26 +1693,28 @@ int launch_attn_rows(RowsAttn &a, hipStream_t s) {
 }
 
 // `part` holds attn_partial_floats(S, rows, n_q, n_kv, hd) floats when a matrix-core path
-// applies, zeroed before its first use (null: k_attn_rows with one chunk, or the plain kernel); `cnt` (when given) replaces its counters.  With `gate`
-// ([rows][n_q]) each head's result is multiplied by softplus of its gate.
+// applies (null: k_attn_rows with one chunk, or the plain kernel), `cnt` ATTN_COUNTERS
+// counters, zeroed before their first use.  With `gate` ([rows][n_q]) each head's result is
+// multiplied by softplus of its gate.
 int run_attention(const float *q, const float *k0, const float *v0, uint32_t n0, const float *k1, const float *v1,
                   uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_kv, uint32_t hd, uint32_t qpos0, int causal,
-                  float *out, float *part, hipStream_t s, const float *gate = nullptr, int gmode = 1,
-                  const GateJob *gj = nullptr, uint32_t *cnt = nullptr) {
+                  float *out, float *part, uint32_t *cnt, hipStream_t s, const float *gate = nullptr, int gmode = 1,
+                  const GateJob *gj = nullptr) {
     const float scale = 1.0f / sqrtf((float)hd);  // src/dflash.rs:1173
     const uint32_t G = n_q / n_kv;
     const bool al = aligned16_ptr(q) && aligned16_ptr(k0) && aligned16_ptr(v0) &&
                     (!k1 || (aligned16_ptr(k1) && aligned16_ptr(v1)));
-    if (part && hd == AHD && rows * G <= AQ && al && rows * G > ADQ) {
+    const bool counted = n_kv <= ATTN_COUNTERS / (AQ / AQG);
+    if (part && hd == AHD && rows * G <= AQ && al && rows * G > ADQ && counted) {
         const uint32_t ngq = (rows * G + AQG - 1) / AQG, groups = n_kv * ngq, nch = attn_split_chunks(S, groups);
         SplitAttn a{};
         a.q = q, a.k0 = k0, a.v0 = v0, a.k1 = k1, a.v1 = v1;
         a.n0 = n0, a.S = S, a.rows = rows, a.n_q = n_q, a.n_kv = n_kv, a.qpos0 = qpos0, a.ngq = ngq, a.nch = nch;
         a.causal = causal, a.gmode = gmode, a.scale = scale;
-        a.part_o = part + attn_cnt_floats(n_kv);
+        a.part_o = part;
         a.part_ml = a.part_o + (size_t)groups * nch * AQG * AHD;
         a.gbuf = a.part_ml + (size_t)groups * nch * AQG * 2;
-        a.cnt = cnt ? cnt : reinterpret_cast<uint32_t *>(part);
+        a.cnt = cnt;
         a.out = out, a.gate = gate, a.gj = gj ? *gj : GateJob{};
         const uint32_t R = n_kv * nch;
         hipLaunchKernelGGL(k_attn_split, dim3((R + 7) / 8 * 8 * ngq), dim3(256), 0, s, a);
@@ -1721,7 +1724,6 @@ int run_attention(const float *q, const float *k0, const float *v0, uint32_t n0,
         // Few queries: the chunks cover the context; a short run of positions after it
         // (the block's own keys in k1) is attended by the combine, so that the chunk
         // grid does not spill a few workgroups into a second round.
-        part += attn_cnt_floats(n_kv);
         const uint32_t T = k1 && S > n0 && S - n0 <= ATAIL ? S - n0 : 0, Sc = T ? n0 : S;
         const uint32_t nch = (Sc + ACH - 1) / ACH;
         float *part_ml = part + (size_t)n_kv * nch * AQ * AHD;
@@ -1739,14 +1741,15 @@ int run_attention(const float *q, const float *k0, const float *v0, uint32_t n0,
         gate = gj->out;
     }
     const uint64_t ngq = ((uint64_t)rows * G + RQB - 1) / RQB;
-    if ((uint64_t)rows * n_q <= 0x7FFFFFFFu && attn_rows_ok(S, rows * G, hd) && al && aligned16_ptr(out) &&
+    if ((uint64_t)rows * n_q <= 0x7FFFFFFFu &&
+        (attn_rows_ok(S, rows * G, hd) || (S && hd == AHD && !counted)) && al && aligned16_ptr(out) &&
         ngq * n_kv <= 0x1000000u) {
         RowsAttn a{};
         a.q = q, a.k0 = k0, a.v0 = v0, a.k1 = k1, a.v1 = v1;
         a.n0 = n0, a.S = S, a.rows = rows, a.n_q = n_q, a.n_kv = n_kv, a.qpos0 = qpos0, a.ngq = (uint32_t)ngq;
         a.causal = causal, a.gmode = gmode, a.scale = scale, a.out = out, a.gate = gate;
         a.nch = part ? rows_chunks(S, n_kv * a.ngq) : 1;
-        a.part_o = part ? part + attn_cnt_floats(n_kv) : nullptr;
+        a.part_o = part;
         a.part_ml = part ? a.part_o + (size_t)n_kv * a.ngq * a.nch * RQB * hd : nullptr;
         return hd == 64 ? launch_attn_rows<64>(a, s) : hd == 256 ? launch_attn_rows<256>(a, s) : launch_attn_rows<AHD>(a, s);
     }
@@ -2032,7 +2035,7 @@ int forward(const lg_dflash_model *md, const FwdLayout &W, const float *features
         // causal attention over [context; injected; tokens] (src/dflash.rs:945-954), each head
         // scaled by softplus of its gate (src/dflash.rs:956-959)
         LG_TRY(run_attention(q, L.k_ctx, L.v_ctx, ctx_len, W.kk, W.vv, ctx_len + 2 * m, m, H, KV, HD, ctx_len + m, 1,
-                             W.att, W.part, s, gate, 1, nullptr, static_cast<uint32_t *>(W.pws)));
+                             W.att, W.part, static_cast<uint32_t *>(W.pws), s, gate));
         LG_TRY(proj(W, W.att, L.attn_output, L.attn_output_type, x, QD, E, m, s, x));  // x += o_proj
         // SwiGLU FFN (src/dflash.rs:962-968)
         LG_TRY(run_rmsnorm(x, L.ffn_norm, W.h, E, m, 1, E, hp.rms_eps, s));
@@ -2125,7 +2128,7 @@ int forward_folded(const lg_dflash_model *md, const FwdLayout &W, const float *f
             q = W.q + (uint64_t)m * QD;
             gate = W.gate + (uint64_t)m * H;
             LG_TRY(run_attention(q, L.k_ctx, L.v_ctx, ctx_len, W.kk, W.vv, ctx_len + 2 * m, m, H, KV, HD, ctx_len + m,
-                                 1, W.att, W.part, s, gate, 1, nullptr, static_cast<uint32_t *>(W.pws)));
+                                 1, W.att, W.part, static_cast<uint32_t *>(W.pws), s, gate));
         } else if (qkf && kvq && L.attn_gate_type == LG_Q4_K) {
             BatchJob jb[3] = {{L.attn_k, W.kk, nullptr, KVD}, {L.attn_v, W.vv, nullptr, KVD},
                               tok_rows({L.attn_q, W.q, nullptr, QD}, m)};
@@ -2138,7 +2141,7 @@ int forward_folded(const lg_dflash_model *md, const FwdLayout &W, const float *f
             gj = {ny, static_cast<const uint8_t *>(L.attn_gate), W.gate + (uint64_t)m * H, H, E, m * H, (m * H + 3) / 4,
                   W.ssa, cols_a, eps};
             LG_TRY(run_attention(q, L.k_ctx, L.v_ctx, ctx_len, W.kk, W.vv, ctx_len + 2 * m, m, H, KV, HD, ctx_len + m,
-                                 1, W.att, W.part, s, nullptr, 1, &gj, static_cast<uint32_t *>(W.pws)));
+                                 1, W.att, W.part, static_cast<uint32_t *>(W.pws), s, nullptr, 1, &gj));
         } else {
             if (kvq && L.attn_k_type == L.attn_gate_type) {
                 const BatchJob jb[4] = {{L.attn_k, W.kk, nullptr, KVD}, {L.attn_v, W.vv, nullptr, KVD},
@@ -2173,7 +2176,7 @@ int forward_folded(const lg_dflash_model *md, const FwdLayout &W, const float *f
                                     qk_job(q, L.attn_q_norm, q, H, ctx_len + m, m), W.freq, HD, hp.rope_dim,
                                     hp.qk_eps, s, gj));
             LG_TRY(run_attention(q, L.k_ctx, L.v_ctx, ctx_len, W.kk, W.vv, ctx_len + 2 * m, m, H, KV, HD, ctx_len + m,
-                                 1, W.att, W.part, s, gate, 1, nullptr, static_cast<uint32_t *>(W.pws)));
+                                 1, W.att, W.part, static_cast<uint32_t *>(W.pws), s, gate));
         }
         // x += o_proj, writing x ffn_norm and the sums of x^2 for the FFN norm (src/dflash.rs:960-962)
         const uint32_t cols_b = proj_batch_norm_cols(L.attn_output_type, QD, E, m);
@@ -2255,10 +2258,13 @@ uint64_t glue_attn_partial_bytes(uint32_t seq_len, uint32_t n_q, uint32_t n_kv, 
     return attn_partial_floats(seq_len, 1, n_q, n_kv, head_dim) * 4;
 }
 
+uint64_t glue_attn_counter_bytes() { return (uint64_t)ATTN_COUNTERS * 4; }
+
 int glue_attention(const float *q, const float *k, const float *v, uint32_t seq_len, uint32_t q_pos, uint32_t n_q,
-                   uint32_t n_kv, uint32_t head_dim, float *out, float *part, hipStream_t s, const float *gate) {
-    return run_attention(q, k, v, seq_len, nullptr, nullptr, seq_len, 1, n_q, n_kv, head_dim, q_pos, 1, out, part, s,
-                         gate, 2);
+                   uint32_t n_kv, uint32_t head_dim, float *out, float *part, uint32_t *cnt, hipStream_t s,
+                   const float *gate) {
+    return run_attention(q, k, v, seq_len, nullptr, nullptr, seq_len, 1, n_q, n_kv, head_dim, q_pos, 1, out, part, cnt,
+                         s, gate, 2);
 }
 
 bool glue_attention_token_ok(uint32_t head_dim, uint32_t n_q, uint32_t n_kv, uint32_t rope_dim) {
@@ -2276,7 +2282,7 @@ int glue_attention_token(const float *q, const float *qn_w, const float *kn_w, c
     t.q = q, t.qn_w = qn_w, t.kn_w = kn_w, t.freq = freq, t.rope = rope_dim ? 1u : 0u, t.pos = pos, t.eps = eps;
     t.scale = 1.0f / sqrtf((float)head_dim);  // src/dflash.rs:1173
     t.k = k, t.v = v, t.S = seq_len, t.n_q = n_q, t.n_kv = n_kv, t.nch = (seq_len + ACH - 1) / ACH;
-    t.part_o = part + attn_cnt_floats(n_kv);
+    t.part_o = part;
     t.part_ml = part + (size_t)n_kv * t.nch * AQ * AHD;
     hipLaunchKernelGGL(k_attn_token, dim3(t.nch, n_kv), dim3(256), 0, s, t);
     LG_TRY(after_launch("attention_token", s));
@@ -2370,27 +2376,26 @@ int lg_dispatch_mha_attn(const float *q, const float *k_seq, const float *v_seq,
         LG_EXTENT(v_seq, (uint64_t)seq_len * n_kv_heads * head_dim * 4, name);
     }
     hipStream_t s = (hipStream_t)stream;
-    float *part = nullptr;
+    // BUF_ATTN: the counters, then the partials
+    uint32_t *cnt = nullptr;
     const uint32_t G = n_q_heads / n_kv_heads;
+    const uint64_t bytes = ((uint64_t)ATTN_COUNTERS + attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim)) * 4;
     if (head_dim == AHD && rows * G <= AQ && seq_len) {
-        void *p = nullptr;
         BufLease lease;
-        LG_TRY(stream_buffer(BUF_ATTN, s, attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim) * 4, lease,
-                             "lg_dispatch_mha_attn"));
-        p = lease.buf->ptr;
-        part = static_cast<float *>(p);
+        LG_TRY(stream_buffer(BUF_ATTN, s, bytes, lease, name));
+        cnt = static_cast<uint32_t *>(lease.buf->ptr);
     } else if (rows_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim)) {
         // k_attn_rows splits the sequence when there is a workspace for its partials, and
         // takes it whole where none can be had (a capture before any such call)
         BufLease lease;
-        if (stream_buffer(BUF_ATTN, s, attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim) * 4, lease,
-                          name) == LG_OK)
-            part = static_cast<float *>(lease.buf->ptr);
+        if (stream_buffer(BUF_ATTN, s, bytes, lease, name) == LG_OK)
+            cnt = static_cast<uint32_t *>(lease.buf->ptr);
         else
             clear_error();
     }
+    float *part = cnt ? reinterpret_cast<float *>(cnt + ATTN_COUNTERS) : nullptr;
     return run_attention(q, k_seq, v_seq, seq_len, nullptr, nullptr, seq_len, rows, n_q_heads, n_kv_heads, head_dim,
-                         q_pos, causal, out, part, s);
+                         q_pos, causal, out, part, cnt, s);
 }
 
 // dispatch_gate_mul / the softplus gate (src/dflash.rs:1236-1266, 956-959):

@@ -235,12 +235,14 @@ int glue_qk_norm_rope2(const float *q, const float *wq, float *q_out, uint32_t n
                        float *k_out, uint32_t n_kv, uint32_t head_dim, uint32_t rope_dim, uint32_t pos,
                        const float *freq, float eps, hipStream_t s);
 // Causal attention of one query row at q_pos over seq_len keys/values; `part` holds
-// glue_attn_partial_bytes(seq_len, n_q, n_kv, head_dim) bytes (or is null: the plain kernel).  With
-// `gate` ([n_q]) each head's result is multiplied by log(1 + exp(gate[h]))
-// (kernels/gate_attn.comp).
+// glue_attn_partial_bytes(seq_len, n_q, n_kv, head_dim) bytes (or is null: kernels that need
+// none), `cnt` glue_attn_counter_bytes() of arrival counters that are zero between calls, at
+// a place that no other data takes.  With `gate` ([n_q]) each head's result is multiplied by
+// log(1 + exp(gate[h])) (kernels/gate_attn.comp).
 uint64_t glue_attn_partial_bytes(uint32_t seq_len, uint32_t n_q, uint32_t n_kv, uint32_t head_dim);
+uint64_t glue_attn_counter_bytes();
 int glue_attention(const float *q, const float *k, const float *v, uint32_t seq_len, uint32_t q_pos, uint32_t n_q,
-                   uint32_t n_kv, uint32_t head_dim, float *out, float *part, hipStream_t s,
+                   uint32_t n_kv, uint32_t head_dim, float *out, float *part, uint32_t *cnt, hipStream_t s,
                    const float *gate = nullptr);
 // One token's attention step over seq_len keys/values: QK-norm + NeoX RoPE at `pos`
 // of the query heads and of key row seq_len - 1 (normed in place in k), the

@@ -23,6 +23,7 @@ constexpr uint32_t TABLE_FLOATS = 128;  // rope_dim <= head_dim <= 256
 
 struct TgtLayout {
     float *x, *nx, *q, *k, *v, *att, *gate, *g, *u, *o, *freq, *freq_swa, *part, *x2;
+    uint32_t *cnt;  // the attention's arrival counters
     uint64_t total;
 };
 
@@ -40,9 +41,11 @@ uint64_t layout(const lg_target_model *md, uint32_t seq_len, uint8_t *base, TgtL
                                glue_attn_partial_bytes(seq_len, (uint32_t)H, hp.n_kv_heads, hp.head_dim) / 4, E};
     float **dst[] = {&L.x, &L.nx, &L.q, &L.k, &L.v, &L.att, &L.gate, &L.g, &L.u, &L.o, &L.freq, &L.freq_swa, &L.part,
                      &L.x2};
-    // the two RoPE tables first, at fixed offsets whatever seq_len is, so that an
-    // uploaded table stays valid across calls
-    uint64_t off = 0;
+    // the attention's counters and the two RoPE tables first, at fixed offsets whatever the
+    // model and seq_len are, so that the counters stay zero and an uploaded table valid
+    // across calls
+    L.cnt = reinterpret_cast<uint32_t *>(base);
+    uint64_t off = glue_attn_counter_bytes();
     const int order[] = {10, 11, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 12};
     for (int i : order) {
         *dst[i] = reinterpret_cast<float *>(base + off);
@@ -222,7 +225,7 @@ int forward_in(const lg_target_model *md, const TgtLayout &W, const float *input
         } else {
             LG_TRY(glue_qk_norm_rope2(W.q, L.attn_q_norm, W.q, H, W.k, L.attn_k_norm, kdst, KV, HD, rd, pos, freq,
                                       hp.qk_eps, s));
-            LG_TRY(glue_attention(W.q, kseq, vseq, seq, seq - 1, H, KV, HD, W.att, W.part, s,
+            LG_TRY(glue_attention(W.q, kseq, vseq, seq, seq - 1, H, KV, HD, W.att, W.part, W.cnt, s,
                                   L.attn_gate ? W.gate : nullptr));
         }
         LG_TRY(proj(W.att, L.attn_output, L.attn_output_type, W.o, QD, E, s));
@@ -295,7 +298,7 @@ int forward(const lg_target_model *md, const TgtLayout &W, const float *input, c
         LG_TRY(glue_qk_norm_rope2(W.q, L.attn_q_norm, W.q, H, W.k, L.attn_k_norm, kdst, KV, HD, rd, pos, freq,
                                   hp.qk_eps, s));
         // src/target.rs:466-494: one position (no cache: the token itself) or the cached sequence
-        LG_TRY(glue_attention(W.q, kseq, vseq, seq, seq - 1, H, KV, HD, W.att, W.part, s,
+        LG_TRY(glue_attention(W.q, kseq, vseq, seq, seq - 1, H, KV, HD, W.att, W.part, W.cnt, s,
                               L.attn_gate ? W.gate : nullptr));
         LG_TRY(proj(W.att, L.attn_output, L.attn_output_type, W.o, QD, E, s));
         LG_TRY(glue_add(W.x, W.o, W.x, E, s));
