@@ -1110,6 +1110,14 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
 //         order in which a lane group holds the probabilities of those positions;
 //   S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, each three products of
 //         the parts (hi hi + hi lo + lo hi); queries scaled as K rows are.
+//   P     taken relative to the query's max over this tile, times 2^14, before its split:
+//         the parts' absolute step (2^-24) then lies 2^-38 below the tile's largest weight,
+//         and a tile with weights below 2^-17 of that takes a third part of them.  Relative
+//         to the running max and unscaled, every weight beside a key 17 nats above it (an
+//         attention sink) would be lost: with a zero value row there and 2048 positions,
+//         errors of 7e-4 / 1e-2 / 3e-1 with such a key 9 / 12 / 16 nats above the others'
+//         largest; here 6e-7 / 1.2e-6 / 8e-7, in f32 throughout (k_attn_simple) 4e-6 / 6e-6 /
+//         1.3e-5.  It takes the call below from 29.8 to 31.1 us.
 //
 // The tile after the next one is loaded into registers, the next one converted into the
 // other LDS buffer, while the current one is multiplied: one barrier per tile.  A tile
@@ -1360,18 +1368,24 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
             for (int t = 0; t < DT; t++) Od[t] *= f;
         }
         m = mn;
-        float pv[8];
+        // the tile's weights and sum relative to its own max, ft takes them to the running one
+        const float tu = tmax == -INFINITY ? 0.0f : tmax, ft = __builtin_amdgcn_exp2f(tmax - mu);
+        float pv[8], tsum = 0.0f;
 #pragma unroll
         for (int pt = 0; pt < 2; pt++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                pv[4 * pt + i] = __builtin_amdgcn_exp2f(sv[pt][i] - mu);
-                lsum += pv[4 * pt + i];
+                pv[4 * pt + i] = __builtin_amdgcn_exp2f(sv[pt][i] - tu);
+                tsum += pv[4 * pt + i];
             }
+        lsum = __builtin_fmaf(tsum, ft, lsum);
         const float vm = fmaxf(fmaxf(L.vmx[b][0], L.vmx[b][1]), fmaxf(L.vmx[b][2], L.vmx[b][3]));
         if (__builtin_amdgcn_ballot_w64(vm >= 0x1p-12f && vm < 255.875f)) {  // uniform
             f16x8 ph, pl;
-            f16_parts8(make_float4(pv[0], pv[1], pv[2], pv[3]), make_float4(pv[4], pv[5], pv[6], pv[7]), neg1, ph, pl);
+            const float4 pa = make_float4(pv[0] * 0x1p14f, pv[1] * 0x1p14f, pv[2] * 0x1p14f, pv[3] * 0x1p14f),
+                         pb = make_float4(pv[4] * 0x1p14f, pv[5] * 0x1p14f, pv[6] * 0x1p14f, pv[7] * 0x1p14f);
+            f16_parts8(pa, pb, neg1, ph, pl);
+            const float fx = ft * 0x1p-22f;
 #pragma unroll
             for (int t = 0; t < DT; t++) {
                 const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
@@ -1381,9 +1395,33 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
                 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl, x, 0, 0, 0);
                 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph, x, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i], 0x1p-8f, Od[t][i]);
+                for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i], fx, Od[t][i]);
                 if constexpr (HD > 128)
                     if (t & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            // weights below 2^-17 of the tile's largest: what their parts dropped, as a third one
+            uint32_t least = 0xFFFFFFFFu;  // of bits - 1: a weight of 0 (masked) counts as the largest
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t u = __float_as_uint(pv[i]) - 1;
+                least = u < least ? u : least;
+            }
+            if (__builtin_amdgcn_ballot_w64(least < 0x37000000u - 1)) {  // 2^-17
+                const float pf[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+                f16x8 pr;
+#pragma unroll
+                for (int i = 0; i < 8; i++) pr[i] = (_Float16)(((pf[i] - (float)ph[i]) - (float)pl[i]) * 0x1p24f);
+#pragma unroll
+                for (int t = 0; t < DT; t++) {
+                    const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
+                    const f16x8 vh = *reinterpret_cast<const f16x8 *>(&L.v[b][0][o]);
+                    const f16x8 vl = *reinterpret_cast<const f16x8 *>(&L.v[b][1][o]);
+                    f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, pr, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pr, x, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i] * 0x1p-24f, fx, Od[t][i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         } else {
             for (uint32_t j = 0; j < RPT; j++) {  // the tile's positions: lane group j / 4 % 4, its weight 4 (j / 16) + j % 4
@@ -1391,7 +1429,7 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
                 float w = pv[0];
 #pragma unroll
                 for (uint32_t i = 1; i < 8; i++) w = e == i ? pv[i] : w;
-                w = __shfl(w, (int)(16 * ((j >> 2) & 3u) + l16));
+                w = __shfl(w * ft, (int)(16 * ((j >> 2) & 3u) + l16));
                 const uint32_t p = RPT * tile + j;
                 const bool live = p < a.S && (!a.causal || p <= qpos);
                 const float *vp = kvrow(a.v0, a.v1, p) + 4 * kg;

@@ -29,11 +29,11 @@ def run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal=1):
     return ob.read_f32(q.size).reshape(q.shape)
 
 
-def check(y, want):
+def check(y, want, tol=TOL):
     assert np.all(np.isfinite(y))
     e = float(np.max(np.abs(y - want)) / np.max(np.abs(want)))
     print(f"  |err|inf/|y|inf = {e:.2e}", flush=True)
-    assert e <= TOL
+    assert e <= tol
 
 
 @pytest.mark.parametrize("n_q,n_kv,hd,rows,S,q_pos,causal", [
@@ -96,6 +96,29 @@ def test_attention_rows_range(ctx, case):
         assert np.all(np.isposinf(y[~sees]))
     if case == "masked_nan":  # element by element: only the NaN's own dim, in the rows that see it
         assert np.all(np.isnan(y[5:, 12:16, 7])) and np.all(np.isfinite(np.delete(y, 7, axis=2)))
+
+
+# several tiles a chunk (16 / 8 / 9 on 256 CUs), so that weights meet a running maximum
+SINK_SHAPES = [(64, 64, 64, 3, 2048), (64, 16, 128, 20, 2048), (32, 32, 256, 2, 2304)]
+
+# An exponent below 32 (base 2) is rounded at most three times on its way to a weight, 2^-20
+# each: 3 * 2^-20 * ln 2 of the weight; what the parts of weights and values add lies below.
+WEIGHT_TOL = 2.5e-6
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", SINK_SHAPES)
+@pytest.mark.parametrize("nats", [9, 12, 16])
+def test_attention_rows_sink(ctx, n_q, n_kv, hd, rows, S, nats):
+    """One key far above the others whose value row is zero: the result is made of the
+    small weights alone."""
+    q, K, V = (a.reshape(a.shape[0], -1, hd) for a in inputs(n_q, n_kv, hd, rows, S, 0x5EED0760 + hd))
+    q[:, :, 0], K[:, :, 0] = 2.0, 0.0
+    K[5], V[5] = 0.0, 0.0
+    K[5, :, 0] = (nats + 3.5) * np.sqrt(hd) / 2.0  # the others reach about 3.5
+    q, K, V = q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
+    print(f"attn rows sink hd={hd} {nats} nats", flush=True)
+    want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd)
+    check(run(ctx, q, K, V, n_q, n_kv, hd, S - rows), want, WEIGHT_TOL)
 
 
 def test_attention_rows_first_call_captured(ctx):
