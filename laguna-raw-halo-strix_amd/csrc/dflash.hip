@@ -1105,9 +1105,13 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
 //   K     wavefront w loads rows 8w .. 8w+7 of the tile (8 lanes a row), scales each row
 //         by the power of two 2^e that puts its largest magnitude in [2^14, 2^15) and
 //         stores its f16 parts (f16_parts2) row by row to LDS, with 2^-e;
-//   V     wavefront w loads positions 4w + i and 16 + 4w + i (i < 4), scales by 2^8, and
-//         stores the f16 parts transposed (per dim, 8 positions a 16-byte word), in the
-//         order in which a lane group holds the probabilities of those positions;
+//   V     wavefront w loads dims HD/4 w .. of the tile's rows, lane group g (16 lanes)
+//         positions 4g + i and 16 + 4g + i (i < 4), scales each dim over the tile as a K row,
+//         and stores the f16 parts transposed (per dim, 8 positions a 16-byte word, in the
+//         order in which a lane group holds the weights of those positions), with 2^-e.  A
+//         fixed 2^8 instead lost what lay far below a tile's largest value (4e-6 of a dim
+//         2^-16 below 1) and sent tiles of zeros or beyond [2^-12, 2^8) to the element-wise
+//         path; with the scale per dim the call below takes 31.9 instead of 31.1 us;
 //   S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, each three products of
 //         the parts (hi hi + hi lo + lo hi); queries scaled as K rows are.
 //   P     taken relative to the query's max over this tile, times 2^14, before its split:
@@ -1121,14 +1125,19 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
 //
 // The tile after the next one is loaded into registers, the next one converted into the
 // other LDS buffer, while the current one is multiplied: one barrier per tile.  A tile
-// with a non-finite K or V or a K magnitude (or queries) of 65504 and above (whose row's
-// other elements the f16 parts would lose), or whose V lies outside [2^-12, 2^8) by its
-// largest magnitude, takes that product element by element in f32 from memory (masked
-// positions skipped, so that what lies past the causal limit never reaches a result).
+// with a K or V (or queries) that is not finite or of 65504 and above (beside which the
+// parts of ordinary elements of its row or dim would be lost, of masked positions too) takes
+// that product element by element in f32 from memory (masked positions skipped, so that
+// what lies past the causal limit never reaches a result; rows that no query of the block
+// sees are not read).
+//
+// Kept to about 2^-22 of itself, at worst 2^-39 of the largest: an element of a K row or of a
+// query among that row, of V among its dim's 32 positions in the tile; a weight to 2^-33, at
+// worst 2^-62 of its query's largest in the tile.
 //
 // One wavefront per (row, q head) over the whole sequence (k_attn_simple) reads K and V
 // once per query, one position at a time, and is bound by that chain: 32 rows of 32 / 8
-// heads over 4096 positions 6880 us, here 31 (about 25 and 5.5 for the merge: the loads of
+// heads over 4096 positions 6880 us, here 32 (about 26 and 5.5 for the merge: the loads of
 // the first tiles, eight tiles a workgroup and K and V twice through the L2, one for each
 // 64 of the 128 queries).
 constexpr uint32_t RQB = 64, RPT = 32;  // queries per workgroup, positions per tile
@@ -1139,9 +1148,9 @@ struct RowsLds {
     static constexpr uint32_t KS = HD + 8;  // halves per K row, likewise
     _Float16 k[2][2][RPT * KS];             // [buffer][hi, lo]
     _Float16 v[2][2][HD * RVS];
-    float ke[2][RPT];   // 2^-e of the K rows
-    float vmx[2][4];    // largest |V| of each wavefront's share (NaN: a NaN among them)
-    uint32_t kbad[2][4];
+    float ke[2][RPT];  // 2^-e of the K rows
+    float ve[2][HD];   // 2^-14 2^-e of the V dims
+    uint32_t kbad[2][4], vbad[2][4];
 };
 
 struct RowsAttn {
@@ -1154,11 +1163,19 @@ struct RowsAttn {
     const float *gate;
 };
 
-// 2^e that puts a (finite, nonzero) magnitude in [2^14, 2^15); 1 for zero and non-finite
+// e such that 2^e puts a nonzero magnitude in [2^14, 2^15), at most 112 (2^-14 2^-e is normal);
+// any e for others
 __device__ __forceinline__ int scale_exp(float amax) {
-    if (!(amax > 0.0f && amax <= 3.4028234664e38f)) return 0;
     const int e = 15 - __builtin_amdgcn_frexp_expf(amax);
-    return e < -126 ? -126 : (e > 126 ? 126 : e);
+    return e < 112 ? e : 112;
+}
+__device__ __forceinline__ float pow2(int e) { return __int_as_float((127 + e) << 23); }  // -126 <= e <= 127
+__device__ __forceinline__ float4 mul4(const float4 &v, float f) { return make_float4(v.x * f, v.y * f, v.z * f, v.w * f); }
+
+// acc, or NaN from the first infinite or NaN value on (finite x: x * 0 is 0; a maximum may drop
+// a NaN)
+__device__ __forceinline__ float not_finite4(float acc, const float4 &v) {
+    return __builtin_fmaf(v.w, 0.0f, __builtin_fmaf(v.z, 0.0f, __builtin_fmaf(v.y, 0.0f, __builtin_fmaf(v.x, 0.0f, acc))));
 }
 
 __device__ __forceinline__ float attn_gate(float gv, int gmode) {
@@ -1169,6 +1186,7 @@ template <int HD>
 __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
     constexpr int J = HD / 32, DT = HD / 16, KV4 = HD / 32;  // k steps, dim tiles, float4s of K per thread
     constexpr int DPT = HD / 64;                             // V dims per thread
+    constexpr int PF = HD <= 128 ? 4 : 2;  // dim tiles of V fragments read ahead
     constexpr int SETS = HD <= 128 ? 2 : 1;                  // tiles ahead in registers (256: the register budget)
     constexpr uint32_t KS = RowsLds<HD>::KS;
     extern __shared__ __attribute__((aligned(16))) uint8_t rows_lds[];
@@ -1181,15 +1199,16 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t G = a.n_q / a.n_kv, nq = a.rows * G, kvld = a.n_kv * HD;
     const float neg1 = neg_one();
-    auto kvrow = [&](const float *b0, const float *b1, uint32_t p) {  // positions past S read row S - 1 (masked)
-        const uint32_t pc = p < a.S ? p : a.S - 1;
-        return (pc < a.n0 ? b0 + (uint64_t)pc * kvld : b1 + (uint64_t)(pc - a.n0) * kvld) + h * HD;
-    };
     // the positions this block can see, its tiles, and this chunk's share of them
     const uint32_t qlast = RQB * qg + RQB - 1 < nq ? RQB * qg + RQB - 1 : nq - 1;
     const uint32_t end = a.causal && a.qpos0 + qlast / G + 1 < a.S ? a.qpos0 + qlast / G + 1 : a.S;
     const uint32_t nt = (end + RPT - 1) / RPT, tb = attn_tile0(c, nt, a.nch), te = attn_tile0(c + 1, nt, a.nch);
+    auto kvrow = [&](const float *b0, const float *b1, uint32_t p) {  // positions that none can see read row end - 1 (masked)
+        const uint32_t pc = p < end ? p : end - 1;
+        return (pc < a.n0 ? b0 + (uint64_t)pc * kvld : b1 + (uint64_t)(pc - a.n0) * kvld) + h * HD;
+    };
 
+    const uint32_t vdim = HD / 4 * wave + DPT * l16;  // this thread's V dims
     typedef float vdims __attribute__((ext_vector_type(DPT)));
     f32x4 kr[SETS][KV4];  // native vectors: arrays of HIP's float4 do not always stay in registers
     vdims vr[SETS][8];
@@ -1200,7 +1219,7 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
         for (int j = 0; j < KV4; j++) kr[s][j] = *reinterpret_cast<const f32x4 *>(kp + 64 * (j >> 1) + 4 * (j & 1));
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float *vp = kvrow(a.v0, a.v1, RPT * tile + (i >> 2) * 16 + 4 * wave + (i & 3)) + DPT * lane;
+            const float *vp = kvrow(a.v0, a.v1, RPT * tile + (i >> 2) * 16 + 4 * kg + (i & 3)) + vdim;
             vr[s][i] = *reinterpret_cast<const vdims *>(vp);
         }
     };
@@ -1212,53 +1231,45 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
         mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0xB1, 0xF, 0xF, false)));
         mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x4E, 0xF, 0xF, false)));
         mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x141, 0xF, 0xF, false)));
-        // x - x is 0 unless x is infinite or NaN (v_max3 may drop a NaN)
         float nf = 0.0f;
 #pragma unroll
-        for (int j = 0; j < KV4; j++) {
-            const float4 f = f4(kr[s][j]);
-            nf += ((f.x - f.x) + (f.y - f.y)) + ((f.z - f.z) + (f.w - f.w));
-        }
+        for (int j = 0; j < KV4; j++) nf = not_finite4(nf, f4(kr[s][j]));
         const int e = scale_exp(mx);
+        const float ks = pow2(e);
         const uint32_t row = 8 * wave + (lane >> 3);
 #pragma unroll
         for (int j = 0; j < KV4; j += 2) {
-            float4 x = f4(kr[s][j]), y = f4(kr[s][j + 1]);
-            x = make_float4(__builtin_ldexpf(x.x, e), __builtin_ldexpf(x.y, e), __builtin_ldexpf(x.z, e),
-                            __builtin_ldexpf(x.w, e));
-            y = make_float4(__builtin_ldexpf(y.x, e), __builtin_ldexpf(y.y, e), __builtin_ldexpf(y.z, e),
-                            __builtin_ldexpf(y.w, e));
             f16x8 hi, lo;
-            f16_parts8(x, y, neg1, hi, lo);
+            f16_parts8(mul4(f4(kr[s][j]), ks), mul4(f4(kr[s][j + 1]), ks), neg1, hi, lo);
             const uint32_t o = row * KS + 32 * j + 8 * (lane & 7u);
             *reinterpret_cast<f16x8 *>(&L.k[b][0][o]) = hi;
             *reinterpret_cast<f16x8 *>(&L.k[b][1][o]) = lo;
         }
-        if ((lane & 7u) == 0) L.ke[b][row] = __builtin_ldexpf(1.0f, -e);
+        if ((lane & 7u) == 0) L.ke[b][row] = pow2(-e);
         const uint64_t kb = __builtin_amdgcn_ballot_w64(nf != 0.0f || !(mx < 65504.0f));
-        // V: dims DPT lane .. of this wavefront's eight positions
-        float vm = 0.0f, vn = 0.0f;
+        // V: dims vdim .. vdim + DPT - 1, this lane group's eight positions of the tile
+        float vn = 0.0f, vmax = 0.0f;
+        vdims ve;
 #pragma unroll
         for (int d = 0; d < DPT; d++) {
-            float4 x = make_float4(vr[s][0][d], vr[s][1][d], vr[s][2][d], vr[s][3][d]);
-            float4 y = make_float4(vr[s][4][d], vr[s][5][d], vr[s][6][d], vr[s][7][d]);
-            vm = absmax8(vm, x, y);
-            vn += (((x.x - x.x) + (x.y - x.y)) + ((x.z - x.z) + (x.w - x.w))) +
-                  (((y.x - y.x) + (y.y - y.y)) + ((y.z - y.z) + (y.w - y.w)));
-            x = make_float4(x.x * 256.0f, x.y * 256.0f, x.z * 256.0f, x.w * 256.0f);
-            y = make_float4(y.x * 256.0f, y.y * 256.0f, y.z * 256.0f, y.w * 256.0f);
+            const float4 x = make_float4(vr[s][0][d], vr[s][1][d], vr[s][2][d], vr[s][3][d]);
+            const float4 y = make_float4(vr[s][4][d], vr[s][5][d], vr[s][6][d], vr[s][7][d]);
+            vn = not_finite4(not_finite4(vn, x), y);
+            const float vm = rows4_max(absmax8(0.0f, x, y));
+            vmax = fmaxf(vmax, vm);
+            const int ev = scale_exp(vm);
             f16x8 hi, lo;
-            f16_parts8(x, y, neg1, hi, lo);
-            const uint32_t o = (DPT * lane + d) * RVS + 8 * wave;
+            f16_parts8(mul4(x, pow2(ev)), mul4(y, pow2(ev)), neg1, hi, lo);
+            const uint32_t o = (vdim + d) * RVS + 8 * kg;
             *reinterpret_cast<f16x8 *>(&L.v[b][0][o]) = hi;
             *reinterpret_cast<f16x8 *>(&L.v[b][1][o]) = lo;
+            ve[d] = pow2(-14 - ev);
         }
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) vm = fmaxf(vm, __shfl_xor(vm, o));
-        const uint64_t vb = __builtin_amdgcn_ballot_w64(vn != 0.0f);
+        if (kg == 0) *reinterpret_cast<vdims *>(&L.ve[b][vdim]) = ve;
+        const uint64_t vb = __builtin_amdgcn_ballot_w64(vn != 0.0f || !(vmax < 65504.0f));
         if (lane == 0) {
             L.kbad[b][wave] = kb ? 1u : 0u;
-            L.vmx[b][wave] = vb ? INFINITY : vm;
+            L.vbad[b][wave] = vb ? 1u : 0u;
         }
     };
 
@@ -1284,14 +1295,12 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
             mx = absmax8(mx, f[2 * j], f[2 * j + 1]);
         }
 #pragma unroll
-        for (int j = 0; j < 2 * J; j++) nf += ((f[j].x - f[j].x) + (f[j].y - f[j].y)) + ((f[j].z - f[j].z) + (f[j].w - f[j].w));
+        for (int j = 0; j < 2 * J; j++) nf = not_finite4(nf, f[j]);
         qbad = __builtin_amdgcn_ballot_w64(nf != 0.0f || !(mx < 65504.0f)) != 0;
         mx = rows4_max(mx);
         const int e = scale_exp(mx);
 #pragma unroll
-        for (int j = 0; j < 2 * J; j++)
-            f[j] = make_float4(__builtin_ldexpf(f[j].x, e), __builtin_ldexpf(f[j].y, e), __builtin_ldexpf(f[j].z, e),
-                               __builtin_ldexpf(f[j].w, e));
+        for (int j = 0; j < 2 * J; j++) f[j] = mul4(f[j], pow2(e));
 #pragma unroll
         for (int j = 0; j < J; j++) f16_parts8(f[2 * j], f[2 * j + 1], neg1, qh[j], ql[j]);
         qs = __builtin_ldexpf(a.scale * 1.44269504088896341f, -e);  // scores in base-2 units
@@ -1379,25 +1388,35 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
                 tsum += pv[4 * pt + i];
             }
         lsum = __builtin_fmaf(tsum, ft, lsum);
-        const float vm = fmaxf(fmaxf(L.vmx[b][0], L.vmx[b][1]), fmaxf(L.vmx[b][2], L.vmx[b][3]));
-        if (__builtin_amdgcn_ballot_w64(vm >= 0x1p-12f && vm < 255.875f)) {  // uniform
+        const uint32_t vbad = (L.vbad[b][0] | L.vbad[b][1]) | (L.vbad[b][2] | L.vbad[b][3]);
+        if (__builtin_amdgcn_readfirstlane(vbad) == 0) {
             f16x8 ph, pl;
             const float4 pa = make_float4(pv[0] * 0x1p14f, pv[1] * 0x1p14f, pv[2] * 0x1p14f, pv[3] * 0x1p14f),
                          pb = make_float4(pv[4] * 0x1p14f, pv[5] * 0x1p14f, pv[6] * 0x1p14f, pv[7] * 0x1p14f);
             f16_parts8(pa, pb, neg1, ph, pl);
-            const float fx = ft * 0x1p-22f;
+            auto frag = [&](f16x8 (&f)[2], int t) __attribute__((always_inline)) {
+                const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
+                f[0] = *reinterpret_cast<const f16x8 *>(&L.v[b][0][o]);
+                f[1] = *reinterpret_cast<const f16x8 *>(&L.v[b][1][o]);
+            };
+            f16x8 vf[PF][2];
+#pragma unroll
+            for (int t = 0; t < PF; t++) frag(vf[t], t);
 #pragma unroll
             for (int t = 0; t < DT; t++) {
-                const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
-                const f16x8 vh = *reinterpret_cast<const f16x8 *>(&L.v[b][0][o]);
-                const f16x8 vl = *reinterpret_cast<const f16x8 *>(&L.v[b][1][o]);
-                f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl, x, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph, x, 0, 0, 0);
+                f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t % PF][1], ph, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t % PF][0], pl, x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t % PF][0], ph, x, 0, 0, 0);
+                if (t + PF < DT) frag(vf[t % PF], t + PF);
+                const float4 ve = *reinterpret_cast<const float4 *>(&L.ve[b][16 * t + 4 * kg]);
+                const float fx[4] = {ve.x * ft, ve.y * ft, ve.z * ft, ve.w * ft};
 #pragma unroll
-                for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i], fx, Od[t][i]);
-                if constexpr (HD > 128)
+                for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i], fx[i], Od[t][i]);
+                if constexpr (HD > 128) {
                     if (t & 1) __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
             // weights below 2^-17 of the tile's largest: what their parts dropped, as a third one
             uint32_t least = 0xFFFFFFFFu;  // of bits - 1: a weight of 0 (masked) counts as the largest
@@ -1413,13 +1432,14 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
                 for (int i = 0; i < 8; i++) pr[i] = (_Float16)(((pf[i] - (float)ph[i]) - (float)pl[i]) * 0x1p24f);
 #pragma unroll
                 for (int t = 0; t < DT; t++) {
-                    const uint32_t o = (16 * t + l16) * RVS + 8 * kg;
-                    const f16x8 vh = *reinterpret_cast<const f16x8 *>(&L.v[b][0][o]);
-                    const f16x8 vl = *reinterpret_cast<const f16x8 *>(&L.v[b][1][o]);
-                    f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, pr, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pr, x, 0, 0, 0);
+                    f16x8 f[2];
+                    frag(f, t);
+                    f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[1], pr, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    x = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[0], pr, x, 0, 0, 0);
+                    const float4 ve = *reinterpret_cast<const float4 *>(&L.ve[b][16 * t + 4 * kg]);
+                    const float fx[4] = {ve.x * ft, ve.y * ft, ve.z * ft, ve.w * ft};
 #pragma unroll
-                    for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i] * 0x1p-24f, fx, Od[t][i]);
+                    for (int i = 0; i < 4; i++) Od[t][i] = __builtin_fmaf(x[i] * 0x1p-24f, fx[i], Od[t][i]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }

@@ -121,6 +121,19 @@ def test_attention_rows_sink(ctx, n_q, n_kv, hd, rows, S, nats):
     check(run(ctx, q, K, V, n_q, n_kv, hd, S - rows), want, WEIGHT_TOL)
 
 
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", SINK_SHAPES)
+@pytest.mark.parametrize("top", [0, 12])
+def test_attention_rows_unequal_dims(ctx, n_q, n_kv, hd, rows, S, top):
+    """Value dimensions of very different magnitude, each held to its own largest result."""
+    q, K, V = inputs(n_q, n_kv, hd, rows, S, 0x5EED0780 + hd)
+    scale = np.exp2(top - np.arange(hd) * 37 % 29).astype(np.float32)  # over 28 binary orders
+    V = (V.reshape(S, n_kv, hd) * scale).reshape(S, -1)
+    print(f"attn rows unequal dims hd={hd} from 2^{top}", flush=True)
+    want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd).reshape(-1, hd)
+    y = run(ctx, q, K, V, n_q, n_kv, hd, S - rows).reshape(-1, hd)
+    check(y / scale, want / scale, WEIGHT_TOL)
+
+
 def test_attention_rows_first_call_captured(ctx):
     """A capture on a stream that has no workspace yet: the sequence is taken whole, and
     the graph's result is the eager one's within rounding."""
