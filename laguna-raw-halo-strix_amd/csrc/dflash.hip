@@ -803,8 +803,12 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
 // halves of k step j), P V on v_mfma_f32_16x16x16f16 (halves s = 0..3: positions 4kg +
 // s).  A tile whose K or V (or a query) has a magnitude f16 cannot hold, or whose V is
 // all below 2^-4 (where lo's subnormal floor would show), takes that product in f32 on
-// v_mfma_f32_16x16x4f32 instead (k steps over the same lanes' values).  No LDS for K
-// and V.  The four wavefronts
+// v_mfma_f32_16x16x4f32 instead (k steps over the same lanes' values).  The weights are
+// scaled by 2^14 for their split, so that one is held to 2^-39 of its wavefront's running
+// max (unscaled, 2^-25: with a key 9 / 12 / 16 nats above the others' largest over a zero
+// value row, 2048 positions, errors of 2.6e-4 / 5.5e-3 / 1.3e-1 against 6e-7 / 8e-7 / 1.9e-5
+// here and 4e-6 / 6e-6 / 1.3e-5 in f32 throughout; the block of 16 rows over 2080 positions
+// 15.8 us either way).  No LDS for K and V.  The four wavefronts
 // meet in LDS (one partial per workgroup), the partial goes to the workspace, and the
 // last workgroup of the (h, qg) group to arrive merges the chunks in chunk order,
 // applies the gate and writes the result.  Workgroups sharing (h, c) sit on one XCD
@@ -898,6 +902,7 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
     for (int dt = 0; dt < 8; dt++) Od[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, lsum = 0.0f;  // running max (base-2 units) and sum of the lane's query
     const float sl2 = a.scale * 1.44269504088896341f;
+    float ps = 0x1p14f;  // the unit of Od and of the weights that meet V (not of lsum)
     // One tile: S^T from kr, then kr refilled with tile `next` (two tiles ahead), the
     // softmax, P V from vr, then vr refilled with tile `next`.  Every load is
     // unconditional (past the wavefront's last tile: the last tile again), so that
@@ -959,7 +964,7 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
         for (int b = 0; b < 8; b += 2) vmx = absmax8(vmx, vr[b], vr[b + 1]);
         if (!__builtin_amdgcn_ballot_w64(!(vmx < 65504.0f)) && __builtin_amdgcn_ballot_w64(vmx >= 0.0625f)) {
             f16x4 ph, pl;
-            f16_parts4(pv[0], pv[1], pv[2], pv[3], neg1, ph, pl);
+            f16_parts4(pv[0] * ps, pv[1] * ps, pv[2] * ps, pv[3] * ps, neg1, ph, pl);
 #pragma unroll
             for (int hh = 0; hh < 2; hh++)
 #pragma unroll
@@ -973,13 +978,18 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
                     o = __builtin_amdgcn_mfma_f32_16x16x16f16(vh, ph, o, 0, 0, 0);
                 }
         } else {
+            if (ps != 1.0f && __builtin_amdgcn_ballot_w64(vmx >= 0x1p96f)) {  // the unit back to 1: no overflow by it
+                ps = 1.0f;
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) Od[dt] *= 0x1p-14f;
+            }
 #pragma unroll
             for (int s = 0; s < 4; s++)
 #pragma unroll
                 for (int hh = 0; hh < 2; hh++)
 #pragma unroll
                     for (int cc = 0; cc < 4; cc++)
-                        Od[4 * hh + cc] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(vr[2 * s + hh], cc), pv[s],
+                        Od[4 * hh + cc] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(vr[2 * s + hh], cc), pv[s] * ps,
                                                                               Od[4 * hh + cc], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1008,6 +1018,9 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
         gate_units();
     }
     lsum = lane_add_x32(lane_add_x16(lsum));
+    const float ips = ps == 1.0f ? 1.0f : 0x1p-14f;
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) Od[dt] *= ips;
     // the wavefronts' partials meet in LDS: lane (query l16, kg) holds dims
     // 64hh + 16kg + 4i + cc in Od[4hh + cc][i]
     if (kg == 0) sm[wave][l16] = m, sl[wave][l16] = lsum;

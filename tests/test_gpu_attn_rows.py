@@ -106,16 +106,20 @@ SINK_SHAPES = [(64, 64, 64, 3, 2048), (64, 16, 128, 20, 2048), (32, 32, 256, 2, 
 WEIGHT_TOL = 2.5e-6
 
 
-@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", SINK_SHAPES)
-@pytest.mark.parametrize("nats", [9, 12, 16])
-def test_attention_rows_sink(ctx, n_q, n_kv, hd, rows, S, nats):
+def sink_inputs(n_q, n_kv, hd, rows, S, nats, at):
     """One key far above the others whose value row is zero: the result is made of the
     small weights alone."""
     q, K, V = (a.reshape(a.shape[0], -1, hd) for a in inputs(n_q, n_kv, hd, rows, S, 0x5EED0760 + hd))
     q[:, :, 0], K[:, :, 0] = 2.0, 0.0
-    K[5], V[5] = 0.0, 0.0
-    K[5, :, 0] = (nats + 3.5) * np.sqrt(hd) / 2.0  # the others reach about 3.5
-    q, K, V = q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
+    K[at], V[at] = 0.0, 0.0
+    K[at, :, 0] = (nats + 3.5) * np.sqrt(hd) / 2.0  # the others reach about 3.5
+    return q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", SINK_SHAPES)
+@pytest.mark.parametrize("nats", [9, 12, 16])
+def test_attention_rows_sink(ctx, n_q, n_kv, hd, rows, S, nats):
+    q, K, V = sink_inputs(n_q, n_kv, hd, rows, S, nats, 5)
     print(f"attn rows sink hd={hd} {nats} nats", flush=True)
     want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd)
     check(run(ctx, q, K, V, n_q, n_kv, hd, S - rows), want, WEIGHT_TOL)
@@ -166,3 +170,32 @@ def test_attention_rows_first_call_captured(ctx):
     hip.hipGraphExecDestroy(ge)
     hip.hipGraphDestroy(g)
     s.destroy()
+
+
+# 9 to 64 queries per kv head of 128: 16 to a workgroup, the sequence over its wavefronts
+@pytest.mark.parametrize("n_q,n_kv,rows,S", [(32, 8, 16, 2048), (64, 64, 9, 700)])
+@pytest.mark.parametrize("nats", [9, 12, 16])
+@pytest.mark.parametrize("at", [0, 5, 300])
+def test_attention_groups_sink(ctx, n_q, n_kv, rows, S, nats, at):
+    q, K, V = sink_inputs(n_q, n_kv, 128, rows, S, nats, at)
+    print(f"attn groups sink n_kv={n_kv} {nats} nats at {at}", flush=True)
+    want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, 128)
+    # a weight is held to 2^-39 of the key's where both meet in one wavefront, a tenth of the
+    # positions at most
+    tol = WEIGHT_TOL + 0.1 * 2.0 ** -39 * np.exp(nats + 3.5)
+    check(run(ctx, q, K, V, n_q, n_kv, 128, S - rows), want, tol)
+
+
+def test_attention_groups_huge_value(ctx):
+    """A value of 3e37 beside ordinary ones: no unit of the weights may overflow it."""
+    n_q, n_kv, rows, S = 32, 8, 16, 500
+    q, K, V = inputs(n_q, n_kv, 128, rows, S, 0x5EED07A0)
+    V = V.reshape(S, n_kv, 128)
+    V[100, 3, 17] = 3.0e37
+    V = V.reshape(S, -1)
+    print("attn groups huge value", flush=True)
+    want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, 128)
+    y = run(ctx, q, K, V, n_q, n_kv, 128, S - rows)
+    check(y, want)
+    big = np.abs(want) > 1e30
+    check(y[~big], want[~big])
