@@ -677,9 +677,8 @@ struct RecBuild {
                     w[i] = v[t][i];
                 }
                 if constexpr (XM == 2) w[i] = silu_mul(w[i], u[t][i]);  // kernels/activation.comp:21-28
+                amax = fmaxf(amax, fabsf(w[i]));
             }
-#pragma unroll
-            for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(w[i]));
             amax = row16_max(amax);
             // 2^e puts the chunk's largest magnitude in [2^14, 2^15); a zero or non-finite
             // chunk keeps e = 0 (non-finite values then reach the products as f16 inf / NaN)
@@ -947,62 +946,102 @@ __device__ __forceinline__ void mm_body(const void *x, const float *up, const Mm
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[i][t][r] = 0.0f;
     RecBuild<T0, XM> rb;
-    RecBuild<T1 ? T1 : 1, XM> rb1;  // T1: tokens 32 ..
-    const void *x1 = static_cast<const uint8_t *>(x) + (uint64_t)32 * k * (XM == 1 ? 2 : 4);
-    const uint32_t m0 = T1 ? 32u : m, m1 = T1 ? m - 32 : 1u;
-    rb.load(x, up, m0, k, c0);
-    if constexpr (T1 > 0) rb1.load(x1, up, m1, k, c0);
-    load_w(Wc[0], 0);
-    load_w(Wc[1], 1);
-    // chunk c's record stored, the activations of chunk c + 1 and the weights of chunk c + 2
-    // (into Wn) issued, chunk c (weights Wk) multiplied
-    auto step = [&](uint32_t c, Chunk &Wn, const Chunk &Wk) __attribute__((always_inline)) {
-        const uint32_t b = T1 ? 0u : c & 1u, cn = c0 + (c + 1 < nch ? c + 1 : nch - 1);
-        rb.store(lrec[b], m0);
+    if constexpr (T1 == 0) {
+        rb.load(x, up, m, k, c0);
+        load_w(Wc[0], 0);
+        load_w(Wc[1], 1);
+        // chunk 0 ahead of the loop, so the loop is entered in the state it repeats
+        rb.store(lrec[0], m);
         __syncthreads();
-        rb.load(x, up, m0, k, cn);
+        rb.load(x, up, m, k, c0 + (1 < nch ? 1 : 0));
         __builtin_amdgcn_sched_barrier(0);  // issue order: the activations, then the weights
-        load_w(Wn, c + 2);
+        load_w(Wc[2], 2);
         __builtin_amdgcn_sched_barrier(0);
-        auto passes = [&](const auto &Ws, auto mul) __attribute__((always_inline)) {
-            mul(std::integral_constant<int, T0>{}, lrec[b], Ws, 0);
-            if constexpr (T1 > 0) {
+        auto chunk = [&](const uint4 *rec, const Chunk &Wk) {
+            if constexpr (RAW4) {
+                Q4kChunk<RT> Ws;
+                stage_q4k<RT>(Wk, Ws, lstage + wave * SPW);
+                q4k_chunk<NP, TT, RT, TT>(rec, Ws, acc, 0);
+            } else if constexpr (Q4) {
+                q4k_chunk<NP, TT, RT, TT>(rec, Wk, acc, 0);
+            } else if constexpr (RAW8) {
+                Q80Chunk<RT> Ws;
+                stage_q80<RT>(Wk, Ws, lstage + wave * SPW);
+                q80_chunk<NP, TT, RT, false, TT>(rec, Ws, acc, 0);
+            } else {
+                q80_chunk<NP, TT, RT, TILED, TT>(rec, Wk, acc, 0);
+            }
+        };
+        chunk(lrec[0], Wc[0]);
+        // three chunks per iteration, so the ring's registers are named at compile time
+        // (chunk c in Wc[c % 3]: ci = 1 mod 3)
+        for (uint32_t ci = 1; ci < nch; ci += 3) {
+#pragma unroll
+            for (int h = 0; h < 3; h++) {
+                const uint32_t c = ci + h;
+                if (c >= nch) break;  // uniform
+                rb.store(lrec[c & 1u], m);
+                __syncthreads();
+                rb.load(x, up, m, k, c0 + (c + 1 < nch ? c + 1 : nch - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                load_w(Wc[h], c + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                chunk(lrec[c & 1u], Wc[(h + 1) % 3]);
+            }
+        }
+    } else {
+        RecBuild<T1 ? T1 : 1, XM> rb1;  // tokens 32 ..
+        const void *x1 = static_cast<const uint8_t *>(x) + (uint64_t)32 * k * (XM == 1 ? 2 : 4);
+        const uint32_t m1 = m - 32;
+        rb.load(x, up, 32, k, c0);
+        rb1.load(x1, up, m1, k, c0);
+        load_w(Wc[0], 0);
+        load_w(Wc[1], 1);
+        // both records stored in turn, the activations of chunk c + 1 and the weights of
+        // chunk c + 2 (into Wn) issued, chunk c (weights Wk) multiplied twice
+        auto step = [&](uint32_t c, Chunk &Wn, const Chunk &Wk) __attribute__((always_inline)) {
+            const uint32_t cn = c0 + (c + 1 < nch ? c + 1 : nch - 1);
+            rb.store(lrec[0], 32);
+            __syncthreads();
+            rb.load(x, up, 32, k, cn);
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(Wn, c + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            auto passes = [&](const auto &Ws, auto mul) __attribute__((always_inline)) {
+                mul(std::integral_constant<int, T0>{}, lrec[0], Ws, 0);
                 rb1.store(lrec[1], m1);
                 __syncthreads();
                 rb1.load(x1, up, m1, k, cn);
                 __builtin_amdgcn_sched_barrier(0);
                 mul(std::integral_constant<int, T1>{}, lrec[1], Ws, T0);
+            };
+            auto mul4 = [&](auto tt, const uint4 *rec, const Q4kChunk<RT> &Ws, int ta) __attribute__((always_inline)) {
+                q4k_chunk<NP, decltype(tt)::value, RT, TT>(rec, Ws, acc, ta);
+            };
+            auto mul8 = [&](auto tt, const uint4 *rec, const Q80Chunk<RT> &Ws, int ta) __attribute__((always_inline)) {
+                q80_chunk<NP, decltype(tt)::value, RT, TILED, TT>(rec, Ws, acc, ta);
+            };
+            if constexpr (RAW4) {
+                Q4kChunk<RT> Ws;
+                stage_q4k<RT>(Wk, Ws, lstage + wave * SPW);
+                passes(Ws, mul4);
+            } else if constexpr (Q4) {
+                passes(Wk, mul4);
+            } else if constexpr (RAW8) {
+                Q80Chunk<RT> Ws;
+                stage_q80<RT>(Wk, Ws, lstage + wave * SPW);
+                passes(Ws, mul8);
+            } else {
+                passes(Wk, mul8);
             }
         };
-        auto mul4 = [&](auto tt, const uint4 *rec, const Q4kChunk<RT> &Ws, int ta) __attribute__((always_inline)) {
-            q4k_chunk<NP, decltype(tt)::value, RT, TT>(rec, Ws, acc, ta);
-        };
-        auto mul8 = [&](auto tt, const uint4 *rec, const Q80Chunk<RT> &Ws, int ta) __attribute__((always_inline)) {
-            q80_chunk<NP, decltype(tt)::value, RT, TILED, TT>(rec, Ws, acc, ta);
-        };
-        if constexpr (RAW4) {
-            Q4kChunk<RT> Ws;
-            stage_q4k<RT>(Wk, Ws, lstage + wave * SPW);
-            passes(Ws, mul4);
-        } else if constexpr (Q4) {
-            passes(Wk, mul4);
-        } else if constexpr (RAW8) {
-            Q80Chunk<RT> Ws;
-            stage_q80<RT>(Wk, Ws, lstage + wave * SPW);
-            passes(Ws, mul8);
-        } else {
-            passes(Wk, mul8);
-        }
-    };
-    // chunk 0 ahead of the loop, so the loop is entered in the state it repeats; three
-    // chunks per iteration, so the ring's registers are named at compile time (chunk c in
-    // Wc[c % 3]: ci = 1 mod 3)
-    step(0, Wc[2], Wc[0]);
-    for (uint32_t ci = 1; ci < nch; ci += 3) {
+        step(0, Wc[2], Wc[0]);
+        for (uint32_t ci = 1; ci < nch; ci += 3) {  // as above
 #pragma unroll
-        for (int h = 0; h < 3; h++) {
-            if (ci + h >= nch) break;  // uniform
-            step(ci + h, Wc[h], Wc[(h + 1) % 3]);
+            for (int h = 0; h < 3; h++) {
+                if (ci + h >= nch) break;  // uniform
+                step(ci + h, Wc[h], Wc[(h + 1) % 3]);
+            }
         }
     }
     constexpr int LREC = 2 * T0 * (int)Fr<NP>::U4 * 16;  // bytes
