@@ -270,7 +270,13 @@ int lg_dispatch_qk_norm_rope(const float *x, const float *norm_w, const float *f
 /* dispatch_mha_attn_seq (src/dflash.rs:1158-1194), kernels/mha_attn.comp:
  * out[r][h] = softmax_p(q[r][h] . k_seq[p][kv(h)] / sqrt(head_dim)) v_seq[p][kv(h)]
  * over p < seq_len (and p <= q_pos + r when causal), kv(h) = h * n_kv / n_q.
- * q: [rows][n_q*head_dim], k_seq, v_seq: [seq_len][n_kv*head_dim]. */
+ * q: [rows][n_q*head_dim], k_seq, v_seq: [seq_len][n_kv*head_dim].
+ *
+ * More than 64 query rows * heads per kv head, and head sizes 64 and 256, split the
+ * sequence over workgroups through a stream workspace of at most 17 MB.  Where that cannot
+ * be had -- the stream is being captured and made no such call before, or no memory is left --
+ * they take it whole: the same result within rounding, several times slower over long
+ * sequences.  A graph keeps the form it was captured with. */
 int lg_dispatch_mha_attn(const float *q, const float *k_seq, const float *v_seq, float *out, uint32_t n_q_heads,
                          uint32_t n_kv_heads, uint32_t head_dim, uint32_t seq_len, uint32_t q_pos,
                          uint32_t rows, int causal, void *stream);

@@ -1730,19 +1730,16 @@ size_t rows_partial_floats(uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_k
     return nch > 1 ? groups * nch * RQB * (hd + 2) : 0;
 }
 
+// Floats of the partials of an attention call, for the kernel that its shape goes to; no
+// more for a shorter sequence.
 size_t attn_partial_floats(uint32_t S, uint32_t rows, uint32_t n_q, uint32_t n_kv, uint32_t hd) {
+    if (hd != AHD || (uint64_t)rows * (n_q / n_kv) > AQ) return rows_partial_floats(S, rows, n_q, n_kv, hd);
     const uint32_t nch = (S + ACH - 1) / ACH, cus = (uint32_t)device_cus();
     const size_t decode = (size_t)n_kv * nch * AQ * (AHD + 2);
     // k_attn_split: groups <= 4 n_kv (at most AQ queries per kv head), groups * chunks <= max(CUs, groups)
     const size_t gc = cus > 4 * n_kv ? cus : 4 * n_kv;
     const size_t split = gc * AQG * (AHD + 2) + (size_t)4 * n_kv * AQG;
-    // k_attn_rows: groups * chunks <= CUs, and no more chunks than rows_chunks' limits (the
-    // bound holds for fewer query heads too: a target's layers may differ in them)
-    const uint64_t groups = (uint64_t)n_kv * (((uint64_t)rows * (n_q / n_kv) + RQB - 1) / RQB);
-    const uint64_t cap = (S + RPT - 1) / RPT, wg = groups * (cap < 64 ? cap : 64);
-    const size_t many = hd == 64 || hd == AHD || hd == 256 ? (wg < cus ? wg : cus) * RQB * (hd + 2) : 0;
-    const size_t few = decode > split ? decode : split;
-    return many > few ? many : few;
+    return decode > split ? decode : split;
 }
 
 template <int HD>
@@ -2450,20 +2447,16 @@ int lg_dispatch_mha_attn(const float *q, const float *k_seq, const float *v_seq,
     hipStream_t s = (hipStream_t)stream;
     // BUF_ATTN: the counters, then the partials
     uint32_t *cnt = nullptr;
-    const uint32_t G = n_q_heads / n_kv_heads;
-    const uint64_t bytes = ((uint64_t)ATTN_COUNTERS + attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim)) * 4;
-    if (head_dim == AHD && rows * G <= AQ && seq_len) {
+    const uint64_t floats = attn_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim);
+    if (seq_len && floats) {
         BufLease lease;
-        LG_TRY(stream_buffer(BUF_ATTN, s, bytes, lease, name));
-        cnt = static_cast<uint32_t *>(lease.buf->ptr);
-    } else if (rows_partial_floats(seq_len, rows, n_q_heads, n_kv_heads, head_dim)) {
-        // k_attn_rows splits the sequence when there is a workspace for its partials, and
-        // takes it whole where none can be had (a capture before any such call)
-        BufLease lease;
-        if (stream_buffer(BUF_ATTN, s, bytes, lease, name) == LG_OK)
-            cnt = static_cast<uint32_t *>(lease.buf->ptr);
-        else
-            clear_error();
+        const int st = stream_buffer(BUF_ATTN, s, ((uint64_t)ATTN_COUNTERS + floats) * 4, lease, name);
+        // k_attn_rows splits the sequence when there is a workspace for its partials, and takes
+        // it whole where the stream is being captured and has none, or no memory is left
+        const bool whole = head_dim != AHD || (uint64_t)rows * (n_q_heads / n_kv_heads) > AQ;
+        if (st == LG_OK) cnt = static_cast<uint32_t *>(lease.buf->ptr);
+        else if (whole && (st == LG_EINVAL || st == LG_ENOMEM)) clear_error();
+        else return st;
     }
     float *part = cnt ? reinterpret_cast<float *>(cnt + ATTN_COUNTERS) : nullptr;
     return run_attention(q, k_seq, v_seq, seq_len, nullptr, nullptr, seq_len, rows, n_q_heads, n_kv_heads, head_dim,

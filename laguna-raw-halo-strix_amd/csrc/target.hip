@@ -37,8 +37,12 @@ uint64_t layout(const lg_target_model *md, uint32_t seq_len, uint8_t *base, TgtL
     const lg_target_hparams &hp = md->hp;
     const uint64_t E = hp.n_embd, H = max_q_dim(md), QD = H * hp.head_dim, KVD = (uint64_t)hp.n_kv_heads * hp.head_dim;
     const uint64_t FF = hp.n_ff;
-    const uint64_t floats[] = {E, E, QD, KVD, KVD, QD, H, FF, FF, E, TABLE_FLOATS, TABLE_FLOATS,
-                               glue_attn_partial_bytes(seq_len, (uint32_t)H, hp.n_kv_heads, hp.head_dim) / 4, E};
+    uint64_t part = 0;  // the largest over the layers, which may differ in their query heads
+    for (uint32_t l = 0; l < hp.n_layers; l++) {
+        const uint64_t b = glue_attn_partial_bytes(seq_len, md->layers[l].n_q_heads, hp.n_kv_heads, hp.head_dim);
+        part = b > part ? b : part;
+    }
+    const uint64_t floats[] = {E, E, QD, KVD, KVD, QD, H, FF, FF, E, TABLE_FLOATS, TABLE_FLOATS, part / 4, E};
     float **dst[] = {&L.x, &L.nx, &L.q, &L.k, &L.v, &L.att, &L.gate, &L.g, &L.u, &L.o, &L.freq, &L.freq_swa, &L.part,
                      &L.x2};
     // the attention's counters and the two RoPE tables first, at fixed offsets whatever the

@@ -1,6 +1,8 @@
 """GPU: attention calls of different head counts in turn on one stream.  They share a
 workspace whose arrival counters have to read zero whatever the previous call wrote behind
 them; a group whose counter does not is never written."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -77,3 +79,31 @@ def test_counters_survive_other_models(ctx):
         assert e <= 2e-5  # test_gpu_target's bound
     for m, *_ in models:
         m.free()
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", [(32, 32, 64, 1, 65536), (64, 16, 256, 2, 20000), (8, 1, 128, 9, 200000)])
+def test_workspace_of_long_sequences(ctx, n_q, n_kv, hd, rows, S):
+    """A long sequence takes no more than its partials: a workgroup of 64 queries per CU."""
+    print(f"attention workspace: {n_q}/{n_kv} heads of {hd}, {rows} rows, {S} positions", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    q, o = lh.GpuBuffer(ctx, 4 * rows * n_q * hd), lh.GpuBuffer(ctx, 4 * rows * n_q * hd)
+    kv = [lh.GpuBuffer(ctx, 4 * S * n_kv * hd) for _ in range(2)]
+    for b in (q, *kv):
+        b.fill(0)
+    o.fill(0xFF)
+    ctx.sync()
+    s = lh.Stream()
+    before = free()
+    lh.check(lh.lib().lg_dispatch_mha_attn(q.ptr, kv[0].ptr, kv[1].ptr, o.ptr, n_q, n_kv, hd, S, S - rows, rows, 1, s.ptr))
+    s.sync()
+    used = before - free()
+    print(f"  {used / 1e6:.1f} MB", flush=True)
+    assert not np.any(o.read_f32(rows * n_q * hd))  # weights of equal keys over zero values
+    assert used <= 4 * (256 * 64 * (hd + 2) + 16384) + (4 << 20)  # allocation granularity
+    s.destroy()
