@@ -2,7 +2,8 @@
 f64 oracle.  The kernel takes blocks of 64 queries over tiles of 32 positions, in one
 chunk or several, on f16 parts of its operands (1e-5 of the largest result, as the other
 matrix-core attention: measured below 2e-6); a tile that those parts cannot hold goes
-element by element."""
+element by element.  And the kernels beside it: 16 queries per workgroup (a strong key,
+huge values), one wavefront per query."""
 import ctypes
 
 import numpy as np
@@ -52,6 +53,76 @@ def test_attention_rows(ctx, n_q, n_kv, hd, rows, S, q_pos, causal):
     y = run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal)
     check(y, dfo.attention(q, K, V, q_pos + np.arange(rows), n_q, n_kv, hd, causal=bool(causal)))
     assert np.array_equal(y, run(ctx, q, K, V, n_q, n_kv, hd, q_pos, causal))
+
+
+# two and three, seven and eight, and whole numbers of tiles a chunk (256 CUs): both LDS buffers,
+# tiles loaded ahead, a ragged end
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S", [
+    (32, 8, 64, 32, 1503), (64, 32, 64, 5, 2000), (16, 16, 64, 3, 1024),
+    (32, 8, 256, 32, 1503), (64, 32, 256, 5, 2000), (16, 16, 256, 3, 1024),
+    (32, 8, 128, 32, 1503), (64, 32, 128, 33, 1984),
+])
+def test_attention_rows_tiles(ctx, n_q, n_kv, hd, rows, S):
+    print(f"attn rows tiles n_q={n_q} n_kv={n_kv} hd={hd} rows={rows} S={S}", flush=True)
+    q, K, V = inputs(n_q, n_kv, hd, rows, S, 0x5EED0710 + S)
+    y = run(ctx, q, K, V, n_q, n_kv, hd, S - rows)
+    check(y, dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd))
+    assert np.array_equal(y, run(ctx, q, K, V, n_q, n_kv, hd, S - rows))
+
+
+# positions in the first, second and third tile of a chunk of three (256 CUs: tiles 2, 3, 4)
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("at", [70, 100, 150])
+@pytest.mark.parametrize("case", ["k_wide", "k_ninf", "v_wide", "v_inf", "v_zero"])
+def test_attention_rows_mixed_chunk(ctx, hd, at, case):
+    """A tile for the element-wise path (or of zeros) among others of its chunk."""
+    n_q, n_kv, rows, S = 32, 8, 20, 1503
+    print(f"attn rows mixed chunk hd={hd} at={at}: {case}", flush=True)
+    q, K, V = (a.reshape(a.shape[0], -1, hd) for a in inputs(n_q, n_kv, hd, rows, S, 0x5EED0730))
+    sees = np.ones((rows, n_q, hd), bool)
+    if case == "k_wide":
+        q[:, :, 5] = 0.0
+        K[at, 2, 5] = 7.0e30
+    elif case == "k_ninf":
+        q[:, :, 0] = np.abs(q[:, :, 0]) + 1.0
+        K[at, :, 0] = -np.inf
+    elif case == "v_wide":
+        V[at, 1, 17] = 7.0e4
+    elif case == "v_inf":
+        V[at, 0, 3] = np.inf
+        sees[:, :4, 3] = False
+    else:
+        V[at // 32 * 32:at // 32 * 32 + 32] = 0.0
+    q, K, V = q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
+    y = run(ctx, q, K, V, n_q, n_kv, hd, S - rows).reshape(sees.shape)
+    ko, vo = np.where(np.isneginf(K), -1e30, K), np.where(np.isfinite(V), V, 0.0)
+    with np.errstate(all="ignore"):
+        want = dfo.attention(q, ko, vo, S - rows + np.arange(rows), n_q, n_kv, hd).reshape(sees.shape)
+    check(y[sees], want[sees])
+    if case == "v_inf":
+        assert np.all(np.isposinf(y[~sees]))
+    if case == "v_wide":  # the other dims are held to their own size
+        check(np.delete(y, 17, axis=2), np.delete(want, 17, axis=2))
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,rows,S,off", [
+    (4, 2, 96, 3, 50, 0), (8, 2, 80, 17, 130, 0), (2, 2, 192, 5, 77, 0), (3, 1, 20, 2, 9, 0),
+    (8, 2, 64, 20, 130, 4), (8, 2, 128, 20, 130, 4), (4, 4, 256, 3, 65, 4), (32, 8, 128, 4, 100, 8),
+])
+def test_attention_wavefront_per_query(ctx, n_q, n_kv, hd, rows, S, off):
+    """The plain kernel: other head sizes, and operands that are not 16-byte aligned."""
+    print(f"attn plain n_q={n_q} n_kv={n_kv} hd={hd} rows={rows} S={S} off={off}", flush=True)
+    q, K, V = inputs(n_q, n_kv, hd, rows, S, 0x5EED0750 + S)
+    bufs = []
+    for a in (q, K, V, np.zeros_like(q)):
+        b = lh.GpuBuffer(ctx, a.nbytes + off)
+        b.fill(0xFF)
+        b.upload(np.ascontiguousarray(a, np.float32), off)
+        bufs.append(b)
+    st = lh.lib().lg_dispatch_mha_attn(*(b.ptr + off for b in bufs), n_q, n_kv, hd, S, S - rows, rows, 1, ctx.stream)
+    lh.check(st)
+    y = bufs[3].read_f32(q.size + off // 4)[off // 4:].reshape(q.shape)
+    check(y, dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd))
 
 
 @pytest.mark.parametrize("case", ["k_wide", "k_small", "q_wide", "v_wide", "v_small", "masked_nan", "v_inf", "k_ninf"])

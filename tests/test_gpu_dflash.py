@@ -111,8 +111,8 @@ ATTN_CASES = [
     (16, 2, 128, 1, 130, 129, 1),      # G = 8
     (32, 8, 128, 1, 100, 50, 0),       # non-causal, ragged chunk
     (32, 8, 128, 3, 66, 40, 1),        # G = 4, rows 3: 12 queries, the matrix-core chunks
-    (32, 8, 128, 32, 300, 250, 1),     # rows*G = 128 > 64: wavefront path
-    (4, 2, 64, 3, 50, 40, 1),          # head_dim 64: wavefront path
+    (32, 8, 128, 32, 300, 250, 1),     # rows*G = 128 > 64: 64-query blocks
+    (4, 2, 64, 3, 50, 40, 1),          # head_dim 64: 64-query blocks
     (2, 2, 256, 2, 33, 31, 1),
 ]
 
