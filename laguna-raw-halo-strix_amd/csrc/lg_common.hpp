@@ -91,6 +91,11 @@ int stream_buffer(int purpose, hipStream_t s, uint64_t need, BufLease &lease, co
 // zero.
 int stream_workspace(hipStream_t s, uint64_t need, void **out);
 
+__device__ __forceinline__ float silu_mul(float g, float u) {
+    // kernels/activation.comp:21-28: silu(g) * up, silu(x) = x * (1 / (1 + exp(-x)))
+    return g * (1.0f / (1.0f + expf(-g))) * u;
+}
+
 // 16- and 8-byte loads and stores coherent across the device (sc1: written through to,
 // and read from, the device's coherence point), for partial results that one
 // workgroup writes and another reads back; buffer offsets in bytes, below 2^31.

@@ -151,11 +151,6 @@ struct MmJobs {
     float *part = jobs.j[J_].part;                                                        \
     const uint32_t n = jobs.j[J_].n, bx = blockIdx.x - jobs.j[J_].g0
 
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    // kernels/activation.comp:21-28: silu(g) * up, silu(x) = x * (1 / (1 + exp(-x)))
-    return g * (1.0f / (1.0f + expf(-g))) * u;
-}
-
 // ---- fragment records
 
 // Maximum over each 16-lane row: DPP xor 1, xor 2 (quad_perm), then row_ror 4 and 8.
@@ -1200,7 +1195,8 @@ MmShape mm_shape(int dtype, bool tiled, uint32_t k, uint32_t n, uint32_t m, bool
     if (!q4 && m > 48) {
         // the record of more than 48 f32 rows leaves a CU's LDS to one workgroup: the split whose
         // rounds over the CUs take the fewest chunks, two more for each round's start and finish,
-        // and never more slices (partial sums) than two workgroups per CU make (m = 64 tiles: n = 14336 60.7 -> 54.4 with one slice, n = 4096 24.2 -> 20.9 with four)
+        // and never more slices (partial sums) than two workgroups per CU make (m = 64 tiles:
+        // n = 14336 60.7 -> 54.4 with one slice, n = 4096 24.2 -> 20.9 with four)
         uint32_t best = ~0u;
         for (uint32_t t = 1, most = slices; t <= nb && t <= (most ? most : 1); t++) {
             const uint32_t cost = (cols * t + cus - 1) / cus * ((nb + t - 1) / t + 2);
@@ -1498,7 +1494,8 @@ int proj_batch_multi(const void *x, int x_dtype, const float *up, const BatchJob
             const uint64_t off = (uint64_t)16 * t0 * jb[j].n;
             // a job whose rows below 16 t0 + 16 (three and four tiles: 16 t0 + 32) are not needed
             // skips those tiles
-            const uint32_t tlo = tt >= 2 && !glu && xm == 0 && !jb[j].ss && jb[j].row0 >= 16 * (t0 + (tt == 2 ? 1 : 2)) ? 1u : 0u;
+            const uint32_t skip = 16 * (t0 + (tt == 2 ? 1 : 2));
+            const uint32_t tlo = tt >= 2 && !glu && xm == 0 && !jb[j].ss && jb[j].row0 >= skip ? 1u : 0u;
             jobs.j[j] = {static_cast<const uint8_t *>(jb[j].w), jb[j].c + off, jb[j].res ? jb[j].res + off : nullptr,
                          reinterpret_cast<float *>(pb), jb[j].y, jb[j].yw, jb[j].ss, jb[j].n, groups, jb[j].qkw, tlo};
             if (sh.slices > 1) pb += align256(mm_part_floats(jb[j].n, ml, sh.rt, sh.slices, glu) * 4);

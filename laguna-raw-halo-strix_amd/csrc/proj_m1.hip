@@ -60,11 +60,6 @@ constexpr int M1_RPW_MAX = 8;         // rows per team whose loads are in flight
 // ------------------------------------------------------------------------------------------
 // activations
 
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    // kernels/activation.comp:21-28: silu(g) * up, silu(x) = x * (1 / (1 + exp(-x)))
-    return g * (1.0f / (1.0f + expf(-g))) * u;
-}
-
 // The same with the hardware exp2 and reciprocal (v_exp_f32 of -g log2(e), v_rcp_f32:
 // each about 1 ulp; non-finite g gives what silu_mul gives), for the fused down
 // projections, whose every workgroup stages all of k: a few instructions instead of

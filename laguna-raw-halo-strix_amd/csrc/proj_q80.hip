@@ -26,11 +26,6 @@ constexpr uint32_t QR_K_MAX = 32768;  // 160 KiB of LDS
 
 typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
 
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    // kernels/activation.comp:21-28: silu(g) * up, silu(x) = x * (1 / (1 + exp(-x)))
-    return g * (1.0f / (1.0f + expf(-g))) * u;
-}
-
 template <int R, bool FUSE>
 __global__ __launch_bounds__(QR_WAVES * 64) void k_q80_rows(const float *__restrict__ x, const float *__restrict__ up,
                                                             const uint8_t *__restrict__ w, float *__restrict__ y,
