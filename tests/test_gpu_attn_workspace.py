@@ -58,6 +58,15 @@ def test_counters_survive_other_head_counts(ctx, before):
     s.destroy()
 
 
+def test_more_groups_than_counters(ctx):
+    """4100 kv heads of 9 queries each: more groups than the counters' region is sized for."""
+    print("attention workspace: 4100 kv heads", flush=True)
+    c, s = Call(ctx, 4100, 4100, 128, 9, 12, 0x5EED0C40), lh.Stream()
+    c.run(s)
+    c.run(s)
+    s.destroy()
+
+
 def test_counters_survive_other_models(ctx):
     """Two targets of different widths, 16 query heads on one kv head, in turn on one stream."""
     models = []
