@@ -1134,7 +1134,10 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitAttn a) {
 //         attention sink) would be lost: with a zero value row there and 2048 positions,
 //         errors of 7e-4 / 1e-2 / 3e-1 with such a key 9 / 12 / 16 nats above the others'
 //         largest; here 6e-7 / 1.2e-6 / 8e-7, in f32 throughout (k_attn_simple) 4e-6 / 6e-6 /
-//         1.3e-5.  It takes the call below from 29.8 to 31.1 us.
+//         1.3e-5.  It takes the call below from 29.8 to 31.1 us.  Scores stay products of
+//         powers of two and the matrix results (no rounding) until their distance from the
+//         max is taken, which sl2 = log2(e) / sqrt(HD) scales: rounded at their own size
+//         instead, scores of +-250 cost weights 1.4e-6 rather than 1.0e-6 (HD 64).
 //
 // The tile after the next one is loaded into registers, the next one converted into the
 // other LDS buffer, while the current one is multiplied: one barrier per tile.  A tile
@@ -1316,9 +1319,9 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
         for (int j = 0; j < 2 * J; j++) f[j] = mul4(f[j], pow2(e));
 #pragma unroll
         for (int j = 0; j < J; j++) f16_parts8(f[2 * j], f[2 * j + 1], neg1, qh[j], ql[j]);
-        qs = __builtin_ldexpf(a.scale * 1.44269504088896341f, -e);  // scores in base-2 units
+        qs = pow2(-e);
     }
-    const float qs1 = a.scale * 1.44269504088896341f;
+    const float sl2 = a.scale * 1.44269504088896341f;  // a weight: 2^(sl2 (q . k - the largest))
     f32x4 Od[DT];
 #pragma unroll
     for (int t = 0; t < DT; t++) Od[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -1367,7 +1370,7 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
                     float d = 0.0f;
                     if (sees(p0 + 16 * pt + i))
                         for (uint32_t e = 0; e < (uint32_t)HD; e++) d = __builtin_fmaf(qp[e], kp[e], d);
-                    sv[pt][i] = d * qs1;
+                    sv[pt][i] = d;
                 }
         }
         // masks only where some query of the wavefront does not see all of the tile (uniform;
@@ -1385,20 +1388,20 @@ __global__ __launch_bounds__(256) void k_attn_rows(RowsAttn a) {
         tmax = rows4_max(tmax);
         const float mn = fmaxf(m, tmax), mu = mn == -INFINITY ? 0.0f : mn;
         if (__builtin_amdgcn_ballot_w64(mn != m)) {  // some query's max moved: rescale (2^-inf = 0)
-            const float f = __builtin_amdgcn_exp2f(m - mu);
+            const float f = __builtin_amdgcn_exp2f((m - mu) * sl2);
             lsum *= f;
 #pragma unroll
             for (int t = 0; t < DT; t++) Od[t] *= f;
         }
         m = mn;
         // the tile's weights and sum relative to its own max, ft takes them to the running one
-        const float tu = tmax == -INFINITY ? 0.0f : tmax, ft = __builtin_amdgcn_exp2f(tmax - mu);
+        const float tu = tmax == -INFINITY ? 0.0f : tmax, ft = __builtin_amdgcn_exp2f((tmax - mu) * sl2);
         float pv[8], tsum = 0.0f;
 #pragma unroll
         for (int pt = 0; pt < 2; pt++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                pv[4 * pt + i] = __builtin_amdgcn_exp2f(sv[pt][i] - tu);
+                pv[4 * pt + i] = __builtin_amdgcn_exp2f((sv[pt][i] - tu) * sl2);
                 tsum += pv[4 * pt + i];
             }
         lsum = __builtin_fmaf(tsum, ft, lsum);
@@ -1544,7 +1547,7 @@ __global__ __launch_bounds__(256) void k_attn_rows_merge(RowsAttn a) {
     float M = mc;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
-    const float w = mc == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc - M);
+    const float w = mc == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mc - M) * (a.scale * 1.44269504088896341f));
     const float l = wave_sum(w * ml.y);
     float o[DPT];
 #pragma unroll
