@@ -243,14 +243,16 @@ def test_attention_rows_first_call_captured(ctx):
     s.destroy()
 
 
-@pytest.mark.parametrize("hd,rows,S", [(64, 3, 40), (64, 40, 700), (256, 3, 40), (256, 40, 700)])
+@pytest.mark.parametrize("hd,rows,S", [(64, 3, 40), (64, 40, 700), (256, 3, 40), (256, 40, 700),
+                                       (128, 70, 2000)])
 def test_attention_rows_large_close_scores(ctx, hd, rows, S):
     """Scores of several thousand, exact in f32, half apart: only their differences count."""
     n_q, n_kv = 4, 4
     q, K, V = (a.reshape(a.shape[0], -1, hd) for a in inputs(n_q, n_kv, hd, rows, S, 0x5EED07C0))
     q[:], K[:] = 0.0, 0.0
     q[:, :, 0] = 64.0
-    K[:, :, 0] = (12000.0 + 4.0 * (np.arange(S) % 7)[:, None]) * np.sqrt(hd) / 512.0
+    # of q . k: 64 times a multiple of 2^-8 (heads of 128: their scores lie 0.35 apart)
+    K[:, :, 0] = (12000.0 + 4.0 * (np.arange(S) % 7)[:, None]) * 2.0 ** (np.log2(hd) // 2) / 512.0
     q, K, V = q.reshape(rows, -1), K.reshape(S, -1), V.reshape(S, -1)
     print(f"attn rows large close scores hd={hd} S={S}", flush=True)
     want = dfo.attention(q, K, V, S - rows + np.arange(rows), n_q, n_kv, hd)
