@@ -54,3 +54,24 @@ def test_f32_block_nonfinite_and_unaligned(ctx, off):
     with np.errstate(invalid="ignore"):
         want = x.astype(np.float64) @ w.astype(np.float64).T
     assert np.all(np.isfinite(y[ok])) and np.max(np.abs(y[ok] - want[ok])) < 1e-5
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("k,ops", [(64, 7.5), (512, 10.75)])
+def test_f32_block_rounding(ctx, k, ops, bf16):
+    """The sum's order: 2-norm error of short rows.  In units of k var(x w), the squared partial
+    sums that are rounded add up to `ops`: 4.5 k in chains of eight products, 1 k for each of
+    three pairings of a block's eight chains, and at 512 (two blocks a wavefront, four
+    wavefronts) 1 k and 2.25 k more; each rounding is 2^-25 of its sum at most."""
+    n, m = 200, 16
+    print(f"f32 block rounding k={k} bf16={bf16}", flush=True)
+    w = synth.normal(0x5EED0820 + k, n * k, 0.02).reshape(n, k)
+    u = synth.normal(0x5EED0821 + k, m * k).view(np.uint32) & np.uint32(0xFFFF0000)
+    x = u.view(np.float32).reshape(m, k)
+    xb = lh.upload_bytes(ctx, (u >> 16).astype(np.uint16).view(np.uint8)) if bf16 else lh.upload_f32(ctx, x)
+    wb, cb = lh.upload_f32(ctx, w), lh.GpuBuffer(ctx, 4 * m * n)
+    lh.dispatch_proj_quant_batch(ctx, xb, lh.BF16 if bf16 else lh.F32, wb, cb, k, n, m, lh.F32)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    e = np.linalg.norm(cb.read_f32(m * n).reshape(m, n) - want) / np.linalg.norm(want)
+    print(f"  {e:.2e}", flush=True)
+    assert e <= np.sqrt(ops) * 2.0 ** -25
